@@ -789,50 +789,58 @@ __global__ __launch_bounds__(256) void gnorm_kernel(Q35LinPrefill p) {
         oa[k] = *reinterpret_cast<const float2 *>(p.out + off);
         za[k] = *reinterpret_cast<const float2 *>(p.z + off);
     }
+    float2 y[TT];
 #pragma unroll
     for (int k = 0; k < TT; k++) {
-        const int b = b0 + k;
-        if (b >= p.B) break;
-        const size_t off = ((size_t)b * p.v_heads + h) * VD + 2 * lane;
         const float2 o = oa[k], z = za[k];
         float ss = o.x * o.x + o.y * o.y;
         ss = q35_wave_sum(ss);
-        float2 y;
         {
 #pragma clang fp contract(off)
             const float r = sqrtf(ss * (1.0f / (float)VD) + 1e-6f), ri = 1.0f / r;
-            y.x = o.x * ri * q35_bf2f((uint16_t)(nw & 0xffff)) * (z.x * q35_sigmoid_fast(z.x));
-            y.y = o.y * ri * q35_bf2f((uint16_t)(nw >> 16)) * (z.y * q35_sigmoid_fast(z.y));
+            y[k].x = o.x * ri * q35_bf2f((uint16_t)(nw & 0xffff)) * (z.x * q35_sigmoid_fast(z.x));
+            y[k].y = o.y * ri * q35_bf2f((uint16_t)(nw >> 16)) * (z.y * q35_sigmoid_fast(z.y));
         }
-        if (!p.xw) {
-            *reinterpret_cast<float2 *>(p.out + off) = y;
-            continue;
-        }
-        q35_f16_guard(p.status, Q35_STATUS_GEMM_F16, q35_f16_over(y.x) || q35_f16_over(y.y));
-        /* The chunk GEMM's X operand instead: quad lanes 4k..4k+3 hold word k
-         * of the head's 16 (values 2i, 2i + 1 in quad lane i); every lane of the
-         * quad gathers the word, lane 0 stores its hi granule, lane 1 its lo.
-         * The group sums (64 columns = one half wave) add the same hi + lo. */
-        float w8[8];
-        w8[0] = q35_dpp<0x00>(y.x), w8[1] = q35_dpp<0x00>(y.y);
-        w8[2] = q35_dpp<0x55>(y.x), w8[3] = q35_dpp<0x55>(y.y);
-        w8[4] = q35_dpp<0xAA>(y.x), w8[5] = q35_dpp<0xAA>(y.y);
-        w8[6] = q35_dpp<0xFF>(y.x), w8[7] = q35_dpp<0xFF>(y.y);
-        f16x8 hi, lo;
+        if (!p.xw && b0 + k < p.B)
+            *reinterpret_cast<float2 *>(p.out + ((size_t)(b0 + k) * p.v_heads + h) * VD + 2 * lane) = y[k];
+    }
+    if (!p.xw) return;
+    /* The chunk GEMM's X operand instead: quad lanes 4w..4w+3 hold word w of
+     * the head's 16 (values 2i, 2i + 1 in quad lane i) of every token; quad
+     * lane i gathers token b0 + i's word and stores its granules, so the quad
+     * writes 64 consecutive bytes (the tokens are consecutive operand rows).
+     * The group sums (64 columns = one half wave) add the same hi + lo. */
+    static_assert(TT == 4, "one token a quad lane");
+    const int G = p.v_heads * VD / 64, v = h * (VD / 8) + (lane >> 2), qi = lane & 3;
+    float w8[8];
+    bool over = false;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float v = w8[q35_xw_perm(j)];
-            hi[j] = (_Float16)v;
-            lo[j] = (_Float16)(v - (float)hi[j]);
-        }
-        const _Float16 hx = (_Float16)y.x, hy = (_Float16)y.y;
-        float s = ((float)hx + (float)(_Float16)(y.x - (float)hx)) + ((float)hy + (float)(_Float16)(y.y - (float)hy));
+    for (int k = 0; k < TT; k++) {
+        over = over || q35_f16_over(y[k].x) || q35_f16_over(y[k].y);
+        const float g8[8] = {q35_dpp<0x00>(y[k].x), q35_dpp<0x00>(y[k].y), q35_dpp<0x55>(y[k].x),
+                             q35_dpp<0x55>(y[k].y), q35_dpp<0xAA>(y[k].x), q35_dpp<0xAA>(y[k].y),
+                             q35_dpp<0xFF>(y[k].x), q35_dpp<0xFF>(y[k].y)};
+#pragma unroll
+        for (int j = 0; j < 8; j++) w8[j] = k == 0 || qi == k ? g8[j] : w8[j];
+        const _Float16 hx = (_Float16)y[k].x, hy = (_Float16)y[k].y;
+        float s = ((float)hx + (float)(_Float16)(y[k].x - (float)hx)) +
+                  ((float)hy + (float)(_Float16)(y[k].y - (float)hy));
         s = q35_half_sum(s);
-        const int G = p.v_heads * VD / 64, v = h * (VD / 8) + (lane >> 2);
-        uint8_t *gr = reinterpret_cast<uint8_t *>(p.xw) + q35_xw_granule(b, v, G);
-        if ((lane & 3) == 0) *reinterpret_cast<f16x8 *>(gr) = hi;
-        if ((lane & 3) == 1) *reinterpret_cast<f16x8 *>(gr + Q35_XW_BLK) = lo;
-        if ((lane & 31) == 0) p.xsum[(size_t)(v >> 3) * p.mpad + b] = s;
+        if ((lane & 31) == 0 && b0 + k < p.B) p.xsum[(size_t)(v >> 3) * p.mpad + b0 + k] = s;
+    }
+    /* (tokens past the batch repeat its last row: no new value to check) */
+    q35_f16_guard(p.status, Q35_STATUS_GEMM_F16, over);
+    f16x8 hi, lo;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float x = w8[q35_xw_perm(j)];
+        hi[j] = (_Float16)x;
+        lo[j] = (_Float16)(x - (float)hi[j]);
+    }
+    if (b0 + qi < p.B) {
+        uint8_t *gr = reinterpret_cast<uint8_t *>(p.xw) + q35_xw_granule(b0 + qi, v, G);
+        *reinterpret_cast<f16x8 *>(gr) = hi;
+        *reinterpret_cast<f16x8 *>(gr + Q35_XW_BLK) = lo;
     }
 }
 

@@ -20,14 +20,12 @@
  *
  * Layouts:
  *   xw      (xprep_kernel) per 64-token tile mt and group g, a 16 KB block
- *           at ((mt G + g) 2 + {0: hi, 1: lo}) 8 KB: 64 rows of 128 bytes,
- *           fp16, 8 consecutive k (one nibble word's worth) kept in the
- *           order 0,4,1,5,2,6,3,7, the order in which a word's nibbles become
- *           fp16 pairs (nibbles j and j + 4 moved to bits 6..9 and 22..25,
- *           ORed into 0x3C003C00, give 1 + q_j / 16 and 1 + q_{j+4} / 16);
- *           word j of row r at 16-byte slot
- *           j ^ (r & 7) ^ ((r >> 3) & 1), so that the MFMA operand reads
- *           (32 rows, one word each) hit distinct LDS banks;
+ *           at ((mt G + g) 2 + {0: hi, 1: lo}) 8 KB, fp16: the group's MFMA
+ *           operands as the waves read them, 1 KB each (q35_xw_granule); 8
+ *           consecutive k (one nibble word's worth) kept in the order
+ *           0,4,1,5,2,6,3,7, the order in which a word's nibbles become fp16
+ *           pairs (nibbles j and j + 4 moved to bits 6..9 and 22..25, ORed
+ *           into 0x3C003C00, give 1 + q_j / 16 and 1 + q_{j+4} / 16);
  *   xsum    fp32 [G][Mpad];
  *   sb      (sb_kernel) (16 s, b - 16 s) as [G][Npad], Npad = N rounded up
  *           to 256, zeros past N;
@@ -48,6 +46,8 @@
  * its own loads of the next group
  * before the one barrier a group.  Two workgroups fit a CU (157.5 KB of
  * LDS), two waves a SIMD.
+ * gemm_few_kernel: the same product split over K inside a workgroup, for
+ * chunks of few tokens (few_tokens picks).
  */
 #include "q35_device.h"
 #include "q35_launch.h"
@@ -68,48 +68,54 @@ constexpr int STAGE = OFF_XS + MT * 4; /* 26880 bytes */
 constexpr int NSTAGE = 3;
 constexpr float QSTEP = 16.0f;         /* B = 1 + q / QSTEP */
 
-/* q35_xw_slot: the 16-byte slot of word j of tile row r in its 128-byte X
- * row is distinct over any 8 consecutive rows and, with the row's 128-byte
- * half, over any 16: the operand reads are free of bank conflicts whether
- * the LDS serves 8 lanes over 32 banks or 16 lanes over 64 banks a cycle */
 /* slot of half h (words 4h..4h+3) of tile feature row r in its 32-byte
- * weight row, by the same argument over 4 and 8 consecutive rows */
+ * weight row: distinct over 4 and 8 consecutive rows, so the operand reads are
+ * free of bank conflicts */
 __device__ __forceinline__ int wslot(int r, int h) { return h ^ (((r >> 2) ^ (r >> 3)) & 1); }
 
-/* x rows -> (optional RMSNorm) -> fp16 hi / lo in word order, tiled, and
- * the group sums of hi + lo.  One workgroup per token row (rows >= M: zeros);
- * thread t takes words t, t + 256, ... of the row, XW of them: the
- * instance is picked by K (1 at 2048, the input projections; 2 at 4096, the
- * GQA output projection; 4 up to 8192), so no thread issues loads past the
- * row (at K = 2048 an instance for 8192 issued nine dead loads a thread:
- * range-checked, they read no memory, but each is still issued and waited
- * for).  The norm is an fp32
- * square sum times the hardware rsq (about 1 ulp from the reference's double
- * sum and division, src/attn_qwen.c:142-157, far below the hi / lo split's
- * 22 bits). */
-template <int XW>
-__global__ __launch_bounds__(NT) void xprep_kernel(Q35Mlx4Xprep p) {
-    const int m = blockIdx.x, t = threadIdx.x, lane = t & 63;
+/* x rows -> (optional RMSNorm) -> fp16 hi / lo operands and the group sums of
+ * hi + lo.  One workgroup of NTX threads per 8 token rows: thread t holds
+ * row t % 8, words t / 8 + i NTX / 8, so a wave takes one 64-column group of
+ * 8 rows at a time, reads 256 consecutive bytes of each row and stores
+ * 128-byte lines of the operand image.  Eight words a thread: NTX = 256 up
+ * to K = 2048 (the input projections), 512 up to 4096 (the GQA output
+ * projection), 1024 up to 8192.  Rows at and past M in the last workgroup are
+ * stored as zeros; operand rows after those are never written: an operand
+ * row only reaches its own output row, which is not stored.  The norm is an
+ * fp32 square sum times the hardware rsq (about 1 ulp from the reference's
+ * double sum and division, src/attn_qwen.c:142-157, far below the hi / lo
+ * split's 22 bits). */
+constexpr int XROWS = 8, XWORDS = 8;
+/* sum over the lanes of equal lane % 8, the total in each of them */
+__device__ __forceinline__ float sum_mod8(float v) {
+    v += q35_xor8(v);
+    return q35_psum32(q35_psum16(v));
+}
+template <int NTX>
+__global__ __launch_bounds__(NTX) void xprep_kernel(Q35Mlx4Xprep p) {
+    const int t = threadIdx.x, lane = t & 63, r = t & 7;
+    const int m0 = blockIdx.x * XROWS, m = m0 + r;
     const int nw = p.K / 8;
-    const bool live = m < p.M;
-    __shared__ float sred[NT / 64];
+    __shared__ float sred[NTX / 64][XROWS];
 
-    /* the thread's words of the row and of the norm weight, all requested
+    /* the thread's words of its row and of the norm weight, all requested
      * at once as range-checked buffer loads (rows past M, words past K and
      * an absent norm weight read as zeros): the norm and the conversion
      * then work from registers, one memory round trip a workgroup */
+    const int nr = min(XROWS, p.M - m0);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        q35_uniform_ptr(const_cast<float *>(live ? p.x + (size_t)m * p.ldx : p.x)), 0, live ? p.K * 4 : 0,
+        q35_uniform_ptr(const_cast<float *>(p.x + (size_t)m0 * p.ldx)), 0, ((nr - 1) * p.ldx + p.K) * 4,
         Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<uint16_t *>(p.norm_w)), 0, p.norm_w ? p.K * 2 : 0, Q35_BUF_DW3);
-    float4 xa[XW], xb[XW];
-    uint4 wv[XW];
+    float4 xa[XWORDS], xb[XWORDS];
+    uint4 wv[XWORDS];
 #pragma unroll
-    for (int i = 0; i < XW; i++) {
-        const int v = t + i * NT;
-        xa[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, 32 * v, 0, 0));
-        xb[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, 32 * v + 16, 0, 0));
+    for (int i = 0; i < XWORDS; i++) {
+        const int v = (t >> 3) + i * (NTX / 8);
+        const uint32_t off = v < nw && r < nr ? (uint32_t)(r * p.ldx + 8 * v) * 4 : 0x80000000u;
+        xa[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
+        xb[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off + 16, 0, 0));
         wv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs, 16 * v, 0, 0));
     }
 
@@ -117,21 +123,23 @@ __global__ __launch_bounds__(NT) void xprep_kernel(Q35Mlx4Xprep p) {
     if (p.norm_w) {
         float ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < XW; i++) {
+        for (int i = 0; i < XWORDS; i++) {
             const float e[8] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w, xb[i].x, xb[i].y, xb[i].z, xb[i].w};
 #pragma unroll
             for (int j = 0; j < 8; j++) ss = fmaf(e[j], e[j], ss);
         }
-        ss = q35_wave_sum(ss);
-        if (lane == 0) sred[t >> 6] = ss;
+        ss = sum_mod8(ss);
+        if (lane < XROWS) sred[t >> 6][lane] = ss;
         q35_lds_barrier();
-        ss = (sred[0] + sred[1]) + (sred[2] + sred[3]);
+        ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NTX / 64; i++) ss += sred[i][r];
         ri = __builtin_amdgcn_rsqf(ss * (1.0f / (float)p.K) + 1e-6f);
     }
 #pragma unroll
-    for (int i = 0; i < XW; i++) {
-        const int v = t + i * NT;
-        if (v >= nw) break;   /* nw is a multiple of 8: the 8 lanes of a group (q35_sum8) leave together */
+    for (int i = 0; i < XWORDS; i++) {
+        const int v = (t >> 3) + i * (NTX / 8);
+        if (v >= nw) break;   /* nw is a multiple of 8: a wave's 8 words leave together */
         float e[8] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w, xb[i].x, xb[i].y, xb[i].z, xb[i].w};
         if (p.norm_w) {
             const uint32_t ww[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
@@ -157,9 +165,9 @@ __global__ __launch_bounds__(NT) void xprep_kernel(Q35Mlx4Xprep p) {
         uint8_t *blk = reinterpret_cast<uint8_t *>(p.xw) + q35_xw_granule(m, v, p.K / 64);
         *reinterpret_cast<f16x8_t *>(blk) = hi;
         *reinterpret_cast<f16x8_t *>(blk + XBLK) = lo;
-        /* the group's 8 words are 8 consecutive threads of a wave */
-        s = q35_sum8(s);
-        if ((v & 7) == 0) p.xsum[(size_t)(v >> 3) * p.Mpad + m] = s;
+        /* the group's 8 words of a row are the wave's lanes of equal lane % 8 */
+        s = sum_mod8(s);
+        if (lane < XROWS) p.xsum[(size_t)(v >> 3) * p.Mpad + m] = s;
     }
 }
 
@@ -355,8 +363,7 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(Q35Mlx4Gemm p) {
                 f16x8_t ah[2], al[2];
 #pragma unroll
                 for (int mb = 0; mb < 2; mb++) {
-                    const int r = 32 * mb + c;
-                    const int off = r * 128 + q35_xw_slot(r, 4 * h + ks) * 16;
+                    const int off = ((mb * 4 + ks) * 64 + lane) * 16;
                     ah[mb] = *reinterpret_cast<const f16x8_t *>(S + off);
                     al[mb] = *reinterpret_cast<const f16x8_t *>(S + XBLK + off);
                 }
@@ -417,6 +424,222 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(Q35Mlx4Gemm p) {
         }
 }
 
+/* ---- the same product for chunks of few tokens ----------------------------
+ * gemm_kernel's one workgroup per 64 x 256 tile leaves most of the GPU idle
+ * when a chunk has few tokens: at M = 64 the 12352 projection rows are 49
+ * workgroups and the output projection 8, each walking all of K by itself.
+ * Here a workgroup owns a (32 MB) x (32 NB) tile and its NW waves take the
+ * groups of K in turn (pairs w, w + NW, ...), so a wave's chain is G / NW
+ * groups and nothing is shared between waves: every operand goes from memory
+ * straight into the registers of the wave that multiplies it (X in operand
+ * order, the weight words in the stage order, both whole lines), with no
+ * LDS staging and no barrier in the loop.  The waves' partial tiles meet in
+ * LDS and are added in wave order, so a result does not depend on timing.
+ * The bias term b' xsum is an fp32 MFMA over the wave's group pairs
+ * (v_mfma_f32_32x32x2_f32: one group a lane half) on its own accumulator.
+ * What bounds it: a CU's 64 B a cycle from L2, (MB K 128 + NB K 20) bytes a
+ * workgroup.  Feature tiles are dealt to the XCDs (id mod 8) with the token
+ * tiles of one feature tile behind each other, so an XCD's L2 fetches a
+ * weight tile once. */
+template <int MB, int NB, int NW>
+__global__ __launch_bounds__(64 * NW) void gemm_few_kernel(Q35Mlx4Gemm p, int nft) {
+    const int ntm = (p.M + 32 * MB - 1) / (32 * MB);
+    const int q = blockIdx.x >> 3, mt = q % ntm;
+    int nt = (q / ntm) * 8 + (blockIdx.x & 7);
+    if (nt >= nft) return;                  /* workgroup-uniform */
+    Q35Mlx4GemmJob J = p.jobs[0];
+#pragma unroll
+    for (int j = 1; j < Q35_GEMM_MAX_JOBS; j++) {
+        const int prev = (J.N + 32 * NB - 1) / (32 * NB);
+        if (j < p.njobs && nt >= prev) {
+            nt -= prev;
+            J = p.jobs[j];
+        }
+    }
+    const int n0 = nt * 32 * NB, m0 = mt * 32 * MB;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int h = lane >> 5, c = lane & 31;
+    const int G = p.K / 64;
+    const int npad = (J.N + NTILE - 1) / NTILE * NTILE;
+    constexpr int RS = 32 * NB + 8;         /* row stride: lane halves (rows 4 apart) on different banks */
+    __shared__ __align__(16) float sp[NW][32 * MB * RS];
+
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr(const_cast<uint16_t *>(p.xw)), 0, (int)((size_t)p.Mpad * p.K * 4), Q35_BUF_DW3);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr(const_cast<uint32_t *>(J.vals)), 0, (int)((size_t)npad * p.K / 2), Q35_BUF_DW3);
+    const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr(const_cast<Q35Mlx4SB *>(J.sb)), 0, (int)((size_t)G * npad * 8), Q35_BUF_DW3);
+    const __amdgpu_buffer_rsrc_t ssr = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr(const_cast<float *>(p.xsum)), 0, (int)((size_t)G * p.Mpad * 4), Q35_BUF_DW3);
+    uint32_t mask, one;
+    asm("s_mov_b32 %0, 0x03c003c0" : "=s"(mask));
+    asm("v_mov_b32 %0, 0x3c003c00" : "=v"(one));
+
+    /* one group's operands: X hi and lo, weight words, s' */
+    struct Ops {
+        u32x4_t xh[MB][4], xl[MB][4], wq[NB];
+        float sc[NB];
+    };
+    int wrow[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) {
+        const int rr = (n0 & (NTILE - 1)) + 32 * nb + c;
+        wrow[nb] = (rr * 2 + wslot(rr, h)) * 16;
+    }
+    const int mt64 = m0 / MT, mb0 = (m0 / 32) & 1, tile = n0 / NTILE;
+    auto load = [&](int g, Ops &o) {
+        const int xb = (mt64 * G + g) * (2 * XBLK) + mb0 * (XBLK / 2);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                o.xh[mb][ks] = __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16 + ks * 1024, xb + mb * 4096, 0);
+                o.xl[mb][ks] = __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16 + ks * 1024, xb + XBLK + mb * 4096, 0);
+            }
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+            o.wq[nb] = __builtin_amdgcn_raw_buffer_load_b128(wr, wrow[nb], (tile * G + g) * WBLK, 0);
+            o.sc[nb] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(sr, (32 * nb + c) * 8, (g * npad + n0) * 8, 0));
+        }
+    };
+
+    f32x16_t acc[MB][NB];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[mb][nb][i] = 0.0f;
+
+    auto multiply = [&](const Ops &o) {
+        f16x8_t bf[NB][4];
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) bf[nb][ks] = nib_f16(o.wq[nb][ks], mask, one);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+                f32x16_t tmp;
+#pragma unroll
+                for (int i = 0; i < 16; i++) tmp[i] = 0.0f;
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++) {
+                    tmp = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, o.xh[mb][ks]),
+                                                                 bf[nb][ks], tmp, 0, 0, 0);
+                    tmp = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, o.xl[mb][ks]),
+                                                                 bf[nb][ks], tmp, 0, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[mb][nb][i] = fmaf(o.sc[nb], tmp[i], acc[mb][nb][i]);
+            }
+    };
+    /* this wave's group pairs; an odd G's missing group reads zeros */
+    for (int g = 2 * w; g < G; g += 2 * NW) {
+        float xs[MB], bs[NB];
+        const int gh = g + h;
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+            xs[mb] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                ssr, gh < G ? (gh * p.Mpad + m0 + 32 * mb + c) * 4 : (int)0x80000000, 0, 0));
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+            bs[nb] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                sr, gh < G ? (gh * npad + n0 + 32 * nb + c) * 8 + 4 : (int)0x80000000, 0, 0));
+        Ops a, b;
+        const bool two = g + 1 < G;
+        load(g, a);
+        if (MB * NB < 4 && two) load(g + 1, b);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++)
+                acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[mb], bs[nb], acc[mb][nb], 0, 0, 0);
+        multiply(a);
+        if (MB * NB >= 4 && two) load(g + 1, b);
+        if (two) multiply(b);
+    }
+
+    /* the waves' tiles -> LDS; lane rows 32mb + 8(i/4) + 4h + i%4, column 32nb + c */
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                sp[w][(32 * mb + 8 * (i >> 2) + 4 * h + (i & 3)) * RS + 32 * nb + c] =
+                    acc[mb][nb][i];
+    q35_lds_barrier();
+    /* y[m][n] (+= with accumulate), four features a thread (N % 4 == 0) */
+    const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr(J.y + (size_t)m0 * J.ldy + n0), 0,
+        ((min(32 * MB, p.M - m0) - 1) * J.ldy + min(32 * NB, J.N - n0)) * 4, Q35_BUF_DW3);
+    constexpr int N4 = 8 * NB;              /* float4s a row */
+    for (int i = t; i < 32 * MB * N4; i += 64 * NW) {
+        const int r = i / N4, n4 = 4 * (i % N4);
+        /* outside the batch or the job's rows: past the view, dropped */
+        const bool in = m0 + r < p.M && n0 + n4 < J.N;
+        const uint32_t off = in ? (uint32_t)(r * J.ldy + n4) * 4 : 0x80000000u;
+        float4 s = p.accumulate
+                       ? __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(yr, off, 0, 0))
+                       : make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 v = *reinterpret_cast<const float4 *>(&sp[0][r * RS + n4]);
+#pragma unroll
+        for (int k = 1; k < NW; k++) {
+            const float4 u = *reinterpret_cast<const float4 *>(&sp[k][r * RS + n4]);
+            v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
+        }
+        s.x += v.x, s.y += v.y, s.z += v.z, s.w += v.w;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, s), yr, off, 0, 0);
+    }
+}
+
+/* Workgroups of a (32 MB) x (32 NB) tiling. */
+inline int64_t few_tiles(const Q35Mlx4Gemm *p, int MB, int NB) {
+    int64_t n = 0;
+    for (int j = 0; j < p->njobs; j++) n += (p->jobs[j].N + 32 * NB - 1) / (32 * NB);
+    return n * ((p->M + 32 * MB - 1) / (32 * MB));
+}
+
+/* Which kernel a product runs on: 0 gemm_kernel, 1..4 gemm_few_kernel at
+ * 32 x 32, 32 x 64 and 64 x 64 with 8 waves, 64 x 64 with 4.  The smallest
+ * tile whose workgroups are at most one a CU (smaller tiles read X more
+ * often, a second round costs as much as the first); past that two 4-wave
+ * workgroups share a CU; and from 140 64 x 64 x 64 products a CU on,
+ * gemm_kernel, whose workgroups share X through LDS, is faster.  us a launch
+ * (projections 12352 x 2048 | output 2048 x 4096), gemm_kernel -> here:
+ *   M =   32: 40.9 ->  8.3 | 75.6 ->  8.8     M =  256: 42.8 -> 36.9 | 77.2 -> 13.1
+ *   M =   64: 41.3 -> 12.1 | 76.3 ->  8.9     M =  512: 55.0 (66.9)  | 76.0 -> 22.3
+ *   M =  128: 42.0 -> 20.4 | 76.8 ->  9.8     M = 1024: 107.7 (139)  | 78.2 -> 45.8
+ * (in brackets the form that is not taken). */
+inline int few_tokens(const Q35Mlx4Gemm *p) {
+    constexpr int64_t CUS = 256;
+    for (int j = 0; j < p->njobs; j++)
+        if (p->jobs[j].N % 4 != 0) return 0;    /* its stores are four features wide */
+    const int64_t t22 = few_tiles(p, 2, 2);
+    if (t22 * (p->K / 64) > 140 * CUS) return 0;
+    if (few_tiles(p, 1, 1) <= CUS) return 1;
+    if (few_tiles(p, 1, 2) <= CUS) return 2;
+    /* half of the last 64-row tile would be padding, at least a fifth of
+     * the work (M = 96, GQA projections: 14.4 us against 19.5) */
+    if (p->M > 64 && p->M <= 160 && p->M % 64 > 0 && p->M % 64 <= 32) return 2;
+    return t22 <= CUS ? 3 : 4;
+}
+
+template <int MB, int NB, int NW>
+hipError_t launch_few(const Q35Mlx4Gemm *p, hipStream_t stream) {
+    int64_t nft = 0;
+    for (int j = 0; j < p->njobs; j++) nft += (p->jobs[j].N + 32 * NB - 1) / (32 * NB);
+    const int64_t grid = (nft + 7) / 8 * 8 * ((p->M + 32 * MB - 1) / (32 * MB));
+    if (grid >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_few_kernel<MB, NB, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, stream, *p, (int)nft);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 extern "C" hipError_t q35_mlx4_sb(const uint16_t *scales, const uint16_t *biases, Q35Mlx4SB *sb, int N,
@@ -439,15 +662,17 @@ extern "C" hipError_t q35_mlx4_wt(const uint32_t *vals, uint32_t *wt, int N, int
 }
 
 extern "C" hipError_t q35_mlx4_xprep(const Q35Mlx4Xprep *p, hipStream_t stream) {
-    if (p->K % 64 != 0 || p->K > 8192 || p->Mpad % MT != 0 || p->M > p->Mpad || p->M < 1)
+    if (p->K % 64 != 0 || p->K > 8192 || p->Mpad % MT != 0 || p->M > p->Mpad || p->M < 1 || p->ldx < p->K ||
+        (int64_t)XROWS * p->ldx * 4 >= ((int64_t)1 << 31))
         return hipErrorInvalidValue;
-    const int words = p->K / 8;           /* words of a row, NT a thread-step */
-    if (words <= NT)
-        hipLaunchKernelGGL(xprep_kernel<1>, dim3(p->Mpad), dim3(NT), 0, stream, *p);
-    else if (words <= 2 * NT)
-        hipLaunchKernelGGL(xprep_kernel<2>, dim3(p->Mpad), dim3(NT), 0, stream, *p);
+    const int words = p->K / 8;           /* words of a row, one thread-step holds NTX / 8 of 8 rows */
+    const dim3 grid((p->M + XROWS - 1) / XROWS);
+    if (words <= 256)
+        hipLaunchKernelGGL(xprep_kernel<256>, grid, dim3(256), 0, stream, *p);
+    else if (words <= 512)
+        hipLaunchKernelGGL(xprep_kernel<512>, grid, dim3(512), 0, stream, *p);
     else
-        hipLaunchKernelGGL(xprep_kernel<4>, dim3(p->Mpad), dim3(NT), 0, stream, *p);
+        hipLaunchKernelGGL(xprep_kernel<1024>, grid, dim3(1024), 0, stream, *p);
     return hipGetLastError();
 }
 
@@ -468,6 +693,11 @@ extern "C" hipError_t q35_mlx4_gemm(const Q35Mlx4Gemm *p, hipStream_t stream) {
     }
     tiles *= p->Mpad / MT;
     if (tiles >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+    const int few = few_tokens(p);
+    if (few == 1) return launch_few<1, 1, 8>(p, stream);
+    if (few == 2) return launch_few<1, 2, 8>(p, stream);
+    if (few == 3) return launch_few<2, 2, 8>(p, stream);
+    if (few == 4) return launch_few<2, 2, 4>(p, stream);
     hipLaunchKernelGGL(gemm_kernel, dim3((unsigned)tiles), dim3(NT), 0, stream, *p);
     return hipGetLastError();
 }
