@@ -215,16 +215,66 @@ __device__ __forceinline__ void vprep_block(const Q35GqaPrefill &p, int bx, int 
     }
 }
 
-/* key / value workspace rows that the prep kernel does not write: positions
- * [0, t0) from the bf16 cache and padding positions [t0+B, 32*kbt) as
- * zeros.  Threads cover (kv head, row r of n_rows, dim); row r maps to
- * position r below t0, else to the padding. */
+/* 8 bf16 values -> 8 fp16; over: one is out of fp16 range */
+__device__ __forceinline__ uint4 bf8_to_f16(uint4 x, bool &over) {
+    const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
+    uint32_t r[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float a = __uint_as_float(xs[i] << 16), b = __uint_as_float(xs[i] & 0xffff0000u);
+        over = over || q35_f16_over(a) || q35_f16_over(b);
+        r[i] = (uint32_t)f16_bits(a) | ((uint32_t)f16_bits(b) << 16);
+    }
+    return make_uint4(r[0], r[1], r[2], r[3]);
+}
+
+/* A whole 32-key tile of cached positions (all before t0) into the fp16
+ * workspaces, one workgroup a (tile, kv head).  8 dims of a key are one
+ * 16-byte granule on both sides; a dim row of a 16-position value tile is 32
+ * bytes of the cache and the 32-byte pair of granules 2 ks, 2 ks + 1 of the
+ * workspace row (keys 0-3, 8-11 | 4-7, 12-15).  Every load of a thread goes
+ * out before the first is used.  At 2 bytes a thread (one element of K and of
+ * V, five divisions and a modulo for its place) this took 47 us at 12345
+ * cached positions and 18 at 4032. */
+__device__ __forceinline__ void prefix_tile(const Q35GqaPrefill &p, int kb, int g) {
+    const int t = threadIdx.x;
+    uint4 k[4], v[2][2];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int i = u * 256 + t, c = i >> 5, key = i & 31;
+        k[u] = *reinterpret_cast<const uint4 *>(p.kt + q35_k_index(g, 32 * kb + key, 8 * c, p.t_tiles));
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        const uint4 *src = reinterpret_cast<const uint4 *>(p.vt + q35_v_index(g, 32 * kb + 16 * ks, t, p.t_tiles));
+        v[ks][0] = src[0];
+        v[ks][1] = src[1];
+    }
+    bool over = false;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int i = u * 256 + t, c = i >> 5, key = i & 31;
+        *reinterpret_cast<uint4 *>(p.kw + kw_index(g, p.kbt, 32 * kb + key, 8 * c)) = bf8_to_f16(k[u], over);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+        const uint4 a = bf8_to_f16(v[ks][0], over), b = bf8_to_f16(v[ks][1], over);   /* keys 0-7, 8-15 */
+        *reinterpret_cast<uint4 *>(p.vw + vw_index(g, p.kbt, kb, t, 16 * ks)) = make_uint4(a.x, a.y, b.x, b.y);
+        *reinterpret_cast<uint4 *>(p.vw + vw_index(g, p.kbt, kb, t, 16 * ks + 8)) = make_uint4(a.z, a.w, b.z, b.w);
+    }
+    q35_f16_guard(p.status, Q35_STATUS_GQA_F16, over);
+}
+
+/* workspace rows that no other role writes, element by element: the cached
+ * positions of the tile t0 lies in and the padding positions [t0+B, 32*kbt)
+ * as zeros.  Threads cover (kv head, row r of n_rows, dim); row r maps to
+ * position 32 (t0 / 32) + r below t0, else to the padding. */
 __device__ __forceinline__ void prefix_rows(const Q35GqaPrefill &p, int n_rows, int bx) {
-    const int64_t i = (int64_t)bx * 256 + threadIdx.x;
-    if (i >= (int64_t)p.kv_heads * n_rows * D) return;
-    const int g = (int)(i / ((int64_t)n_rows * D));
-    const int r = (int)((i / D) % n_rows), d = (int)(i % D);
-    const int pos = r < p.t0 ? r : p.t0 + p.B + (r - p.t0);
+    const int i = bx * 256 + (int)threadIdx.x;           /* at most 2 x 62 x 256 */
+    if (i >= p.kv_heads * n_rows * D) return;
+    const int g = i / (n_rows * D), r = (i / D) % n_rows, d = i % D;
+    const int cached = p.t0 & 31;
+    const int pos = r < cached ? p.t0 - cached + r : p.t0 + p.B + (r - cached);
     float kf = 0.0f, vf = 0.0f;
     if (pos < p.t0) {
         kf = q35_bf2f(p.kt[q35_k_index(g, pos, d, p.t_tiles)]);
@@ -235,20 +285,24 @@ __device__ __forceinline__ void prefix_rows(const Q35GqaPrefill &p, int n_rows, 
     p.vw[vw_index(g, p.kbt, pos >> 5, d, v_slot(pos & 31))] = f16_bits(vf);
 }
 
-/* the three set-up passes in one launch (they write disjoint workspace
- * and cache elements; as three launches the two dispatch gaps and the
- * smaller kernels' tails cost about as much as the work): blocks [0, nk)
- * prep_rows, the next nvb * kv_heads blocks vprep_block, the rest
- * prefix_rows.  Every branch is block-uniform, so vprep_block's barrier
- * sees all of its block's threads. */
+/* the set-up passes in one launch (they write disjoint workspace and cache
+ * elements; as separate launches the dispatch gaps and the smaller kernels'
+ * tails cost about as much as the work): blocks [0, nk) prep_rows, the next
+ * nvb * kv_heads blocks vprep_block, then t0 / 32 * kv_heads of prefix_tile,
+ * the rest prefix_rows.  Every branch is block-uniform, so vprep_block's
+ * barrier sees all of its block's threads. */
 __global__ __launch_bounds__(256) void prep_kernel(Q35GqaPrefill p, int nvb, int n_rows) {
-    const int nk = (p.B + 3) / 4, nv = nvb * p.kv_heads, bx = (int)blockIdx.x;
-    if (bx < nk)
+    const int nk = (p.B + 3) / 4, nv = nvb * p.kv_heads, nt = p.t0 >> 5;
+    int bx = (int)blockIdx.x;
+    if (bx < nk) {
         prep_rows(p, bx);
-    else if (bx < nk + nv)
-        vprep_block(p, (bx - nk) % nvb, (bx - nk) / nvb);
-    else
-        prefix_rows(p, n_rows, bx - nk - nv);
+    } else if ((bx -= nk) < nv) {
+        vprep_block(p, bx % nvb, bx / nvb);
+    } else if ((bx -= nv) < nt * p.kv_heads) {
+        prefix_tile(p, bx % nt, bx / nt);
+    } else {
+        prefix_rows(p, n_rows, bx - nt * p.kv_heads);
+    }
 }
 
 /* LDS: per group, two stages of one 32-key block, each the K tile (16 KB,
@@ -741,11 +795,11 @@ extern "C" hipError_t q35_gqa_prefill(const Q35GqaPrefill *pin, hipStream_t stre
     if (p.heads != p.kv_heads * G || p.kv_heads != 2 || p.B < 1 || p.t0 < 0) return hipErrorInvalidValue;
     p.nqb = (p.B + 15) / 16;
     p.kbt = (p.t0 + p.B + 31) / 32;
-    /* value blocks of the new keys, and rows prep_rows / vprep_block leave:
-     * the prefix and the key padding */
+    /* value blocks of the new keys, whole tiles of the prefix, and the rows
+     * those leave: the prefix's last, partial tile and the key padding */
     const int nvb = ((p.t0 + p.B - 1) >> 5) - (p.t0 >> 5) + 1;
-    const int n_rows = p.t0 + (p.kbt * 32 - (p.t0 + p.B));
-    const int64_t nblk = (p.B + 3) / 4 + (int64_t)nvb * p.kv_heads +
+    const int n_rows = (p.t0 & 31) + (p.kbt * 32 - (p.t0 + p.B));
+    const int64_t nblk = (p.B + 3) / 4 + (int64_t)nvb * p.kv_heads + (int64_t)(p.t0 >> 5) * p.kv_heads +
                          ((int64_t)p.kv_heads * n_rows * D + 255) / 256;
     if (nblk > INT32_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(prep_kernel, dim3((unsigned)nblk), dim3(256), 0, stream, p, nvb, n_rows);
