@@ -74,45 +74,50 @@ constexpr float QSTEP = 16.0f;         /* B = 1 + q / QSTEP */
 __device__ __forceinline__ int wslot(int r, int h) { return h ^ (((r >> 2) ^ (r >> 3)) & 1); }
 
 /* x rows -> (optional RMSNorm) -> fp16 hi / lo operands and the group sums of
- * hi + lo.  One workgroup of NTX threads per 8 token rows: thread t holds
- * row t % 8, words t / 8 + i NTX / 8, so a wave takes one 64-column group of
- * 8 rows at a time, reads 256 consecutive bytes of each row and stores
- * 128-byte lines of the operand image.  Eight words a thread: NTX = 256 up
- * to K = 2048 (the input projections), 512 up to 4096 (the GQA output
- * projection), 1024 up to 8192.  Rows at and past M in the last workgroup are
- * stored as zeros; operand rows after those are never written: an operand
- * row only reaches its own output row, which is not stored.  The norm is an
- * fp32 square sum times the hardware rsq (about 1 ulp from the reference's
- * double sum and division, src/attn_qwen.c:142-157, far below the hi / lo
- * split's 22 bits). */
-constexpr int XROWS = 8, XWORDS = 8;
-/* sum over the lanes of equal lane % 8, the total in each of them */
-__device__ __forceinline__ float sum_mod8(float v) {
+ * hi + lo.  One workgroup of NTX threads per XR token rows: thread t holds
+ * row t % XR, words t / XR + i NTX / XR (WT of them), so the lanes of a
+ * 64-column group are 8 XR neighbours, reads are 256 consecutive bytes of each
+ * row and stores 16 XR bytes of the operand image.  XR = 8 stores whole
+ * 128-byte lines, but with few tokens it is few workgroups that convert 8
+ * rows each; launch_xprep has the line.
+ * Rows at and past M in the last workgroup are stored as zeros; operand rows
+ * after those are never written: an operand row only reaches its own output
+ * row, which is not stored.  The norm is an fp32 square sum times the hardware
+ * rsq (about 1 ulp from the reference's double sum and division,
+ * src/attn_qwen.c:142-157, far below the hi / lo split's 22 bits). */
+/* sum over the 8 lanes of one row's words of a group (8 XR neighbouring
+ * lanes, equal lane % XR), the total in each of them */
+template <int XR>
+__device__ __forceinline__ float group_sum(float v) {
+    static_assert(XR == 8 || XR == 4 || XR == 2, "lane patterns of 2, 4 and 8 rows");
     v += q35_xor8(v);
-    return q35_psum32(q35_psum16(v));
+    if constexpr (XR == 8) return q35_psum32(q35_psum16(v));
+    v += q35_dpp<0x124>(v);                /* row_ror:4, on sums of period 8 */
+    if constexpr (XR == 4) return q35_psum16(v);
+    return v + q35_dpp<0x122>(v);          /* row_ror:2, on sums of period 4 */
 }
-template <int NTX>
+template <int NTX, int XR, int WT>
 __global__ __launch_bounds__(NTX) void xprep_kernel(Q35Mlx4Xprep p) {
-    const int t = threadIdx.x, lane = t & 63, r = t & 7;
-    const int m0 = blockIdx.x * XROWS, m = m0 + r;
+    const int t = threadIdx.x, lane = t & 63, r = t % XR;
+    const int m0 = blockIdx.x * XR, m = m0 + r;
     const int nw = p.K / 8;
-    __shared__ float sred[NTX / 64][XROWS];
+    __shared__ float sred[NTX / 64][XR];
 
     /* the thread's words of its row and of the norm weight, all requested
      * at once as range-checked buffer loads (rows past M, words past K and
      * an absent norm weight read as zeros): the norm and the conversion
      * then work from registers, one memory round trip a workgroup */
-    const int nr = min(XROWS, p.M - m0);
+    const int nr = min(XR, p.M - m0);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<float *>(p.x + (size_t)m0 * p.ldx)), 0, ((nr - 1) * p.ldx + p.K) * 4,
         Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<uint16_t *>(p.norm_w)), 0, p.norm_w ? p.K * 2 : 0, Q35_BUF_DW3);
-    float4 xa[XWORDS], xb[XWORDS];
-    uint4 wv[XWORDS];
+    float4 xa[WT], xb[WT];
+    uint4 wv[WT];
 #pragma unroll
-    for (int i = 0; i < XWORDS; i++) {
-        const int v = (t >> 3) + i * (NTX / 8);
+    for (int i = 0; i < WT; i++) {
+        const int v = t / XR + i * (NTX / XR);
         const uint32_t off = v < nw && r < nr ? (uint32_t)(r * p.ldx + 8 * v) * 4 : 0x80000000u;
         xa[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
         xb[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off + 16, 0, 0));
@@ -123,13 +128,15 @@ __global__ __launch_bounds__(NTX) void xprep_kernel(Q35Mlx4Xprep p) {
     if (p.norm_w) {
         float ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < XWORDS; i++) {
+        for (int i = 0; i < WT; i++) {
             const float e[8] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w, xb[i].x, xb[i].y, xb[i].z, xb[i].w};
 #pragma unroll
             for (int j = 0; j < 8; j++) ss = fmaf(e[j], e[j], ss);
         }
-        ss = sum_mod8(ss);
-        if (lane < XROWS) sred[t >> 6][lane] = ss;
+        ss = group_sum<XR>(ss);
+        if constexpr (XR == 2) ss = q35_psum16(ss);
+        if constexpr (XR <= 4) ss = q35_psum32(ss);
+        if (lane < XR) sred[t >> 6][lane] = ss;
         q35_lds_barrier();
         ss = 0.0f;
 #pragma unroll
@@ -137,9 +144,9 @@ __global__ __launch_bounds__(NTX) void xprep_kernel(Q35Mlx4Xprep p) {
         ri = __builtin_amdgcn_rsqf(ss * (1.0f / (float)p.K) + 1e-6f);
     }
 #pragma unroll
-    for (int i = 0; i < XWORDS; i++) {
-        const int v = (t >> 3) + i * (NTX / 8);
-        if (v >= nw) break;   /* nw is a multiple of 8: a wave's 8 words leave together */
+    for (int i = 0; i < WT; i++) {
+        const int v = t / XR + i * (NTX / XR);
+        if (v >= nw) break;   /* nw is a multiple of 8: a group's 8 words leave together */
         float e[8] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w, xb[i].x, xb[i].y, xb[i].z, xb[i].w};
         if (p.norm_w) {
             const uint32_t ww[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
@@ -165,9 +172,8 @@ __global__ __launch_bounds__(NTX) void xprep_kernel(Q35Mlx4Xprep p) {
         uint8_t *blk = reinterpret_cast<uint8_t *>(p.xw) + q35_xw_granule(m, v, p.K / 64);
         *reinterpret_cast<f16x8_t *>(blk) = hi;
         *reinterpret_cast<f16x8_t *>(blk + XBLK) = lo;
-        /* the group's 8 words of a row are the wave's lanes of equal lane % 8 */
-        s = sum_mod8(s);
-        if (lane < XROWS) p.xsum[(size_t)(v >> 3) * p.Mpad + m] = s;
+        s = group_sum<XR>(s);
+        if ((lane & (8 * XR - 1)) < XR) p.xsum[(size_t)(v >> 3) * p.Mpad + m] = s;
     }
 }
 
@@ -661,18 +667,38 @@ extern "C" hipError_t q35_mlx4_wt(const uint32_t *vals, uint32_t *wt, int N, int
     return hipGetLastError();
 }
 
+namespace {
+/* XR rows a workgroup of N1 threads for K <= 2048 (256 words a row), N2 for
+ * K <= 4096, 1024 for K <= 8192, as many words a thread as that takes */
+template <int XR, int N1, int N2>
+void launch_xprep(const Q35Mlx4Xprep *p, hipStream_t stream) {
+    const int words = p->K / 8;
+    const dim3 grid((p->M + XR - 1) / XR);
+    if (words <= 256)
+        hipLaunchKernelGGL((xprep_kernel<N1, XR, 256 * XR / N1>), grid, dim3(N1), 0, stream, *p);
+    else if (words <= 512)
+        hipLaunchKernelGGL((xprep_kernel<N2, XR, 512 * XR / N2>), grid, dim3(N2), 0, stream, *p);
+    else
+        hipLaunchKernelGGL((xprep_kernel<1024, XR, XR>), grid, dim3(1024), 0, stream, *p);
+}
+}  // namespace
+
 extern "C" hipError_t q35_mlx4_xprep(const Q35Mlx4Xprep *p, hipStream_t stream) {
     if (p->K % 64 != 0 || p->K > 8192 || p->Mpad % MT != 0 || p->M > p->Mpad || p->M < 1 || p->ldx < p->K ||
-        (int64_t)XROWS * p->ldx * 4 >= ((int64_t)1 << 31))
+        (int64_t)8 * p->ldx * 4 >= ((int64_t)1 << 31))
         return hipErrorInvalidValue;
-    const int words = p->K / 8;           /* words of a row, one thread-step holds NTX / 8 of 8 rows */
-    const dim3 grid((p->M + XROWS - 1) / XROWS);
-    if (words <= 256)
-        hipLaunchKernelGGL(xprep_kernel<256>, grid, dim3(256), 0, stream, *p);
-    else if (words <= 512)
-        hipLaunchKernelGGL(xprep_kernel<512>, grid, dim3(512), 0, stream, *p);
+    /* us a launch at XR = 2 | 4 | 8 (K = 2048; K = 4096):
+     *   M =   64:  2.9 |  3.8 |  5.5;   3.0 |  4.6 |  8.1
+     *   M =  256:  3.5 |  4.0 |  5.7;   4.4 |  5.1 |  8.5
+     *   M = 1024:  6.3 |  4.9 |  6.5;  10.0 |  7.9 | 10.3
+     *   M = 2048: 10.3 |  7.5 |  8.2;  19.1 | 12.7 | 11.6
+     *   M = 4096: 19.4 | 12.6 | 11.6;  36.7 | 23.0 | 21.5 */
+    if (p->M <= 256)
+        launch_xprep<2, 512, 1024>(p, stream);
+    else if (p->M <= 2048)
+        launch_xprep<4, 512, 1024>(p, stream);
     else
-        hipLaunchKernelGGL(xprep_kernel<1024>, grid, dim3(1024), 0, stream, *p);
+        launch_xprep<8, 512, 512>(p, stream);
     return hipGetLastError();
 }
 

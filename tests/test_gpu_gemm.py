@@ -37,14 +37,15 @@ class Xprep(ctypes.Structure):
 # (M, rows of the jobs, K): 32 x 32 tiles (one token, one group; an odd group
 # count; a ragged width), 32 x 64 (a layer's rows; half-empty last tiles at 96
 # and 160 tokens), 64 x 64 with 8 waves and with 4, the general kernel by work
-# and by a row count that is not a multiple of 4; K past 2048 and 4096 for the
-# wider X preps
+# and by a row count that is not a multiple of 4; K past 2048 and 4096 and M past
+# 256 and 2048 for the X prep's forms
 @pytest.mark.parametrize("M,Ns,K", [
     (1, (32,), 64), (2, (100, 32), 192), (33, (64,), 320), (128, (2048,), 4096),
     (7, (8192, 4096, 32, 32), 2048), (96, (8192, 512, 512), 2048), (160, (2048,), 4096),
     (64, (8192, 4096, 32, 32), 2048), (63, (8192, 512, 512), 1984),
     (129, (8192, 512, 512), 2048), (1000, (2048,), 2112), (449, (8192, 4096, 32, 32), 2048),
-    (5, (99, 64), 128), (9, (68,), 8192)])
+    (5, (99, 64), 128), (9, (68,), 8192),
+    (257, (64,), 2048), (258, (32,), 8192), (2049, (32,), 2048), (2055, (32,), 4096), (2050, (32,), 8192)])
 @pytest.mark.parametrize("accumulate", [0, 1])
 def test_gemm_matches_float64(M, Ns, K, accumulate):
     import torch
