@@ -14,8 +14,9 @@
  * 2. prefix: cache rows of positions before t0 (earlier chunks) into the
  *            fp16 key / value workspaces; zero padding rows (only launched
  *            when there are such rows).
- * 3. attn:   grid = (pairs of 16-position q blocks, kv heads), 8 waves in
- *            two groups of 4.  A group serves the 8 q heads of its kv head
+ * 3. attn:   grid = (pairs of 16-position q blocks, kv heads), or for short
+ *            chunks (q block, span of its keys, kv head) and a merge, 8
+ *            waves in two groups of 4.  A group serves the 8 q heads of its kv head
  *            for one q block (wave w: heads 2w, 2w+1 x 16 positions = 32
  *            columns); group A runs the long block's first key tiles,
  *            group B the short block and then the long block's remaining
@@ -497,13 +498,20 @@ __device__ __forceinline__ void load_q(const Q35GqaPrefill &p, int g, int qb, in
  * and V tiles of tile it+1; for group B the K tile of tile it+1 and the V
  * tile of tile it (which it reads in the next interval), so no stage part
  * is written in an interval in which its group reads it.  Group A issues
- * its loads among its QK MFMAs, group B among its PV MFMAs. */
+ * its loads among its QK MFMAs, group B among its PV MFMAs.
+ * SPLIT, for calls whose pairs leave CUs idle (spans_for): a workgroup
+ * serves one q block over span_tiles key tiles of it, group A the first half
+ * of them and group B the rest, as in the long block above; a block of
+ * several spans leaves its merged (max, sum, O), fp32, to
+ * span_merge_kernel. */
+template <bool SPLIT>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kernel(Q35GqaPrefill p) {
     /* 1-D grid over (pair, kv head).  Workgroups go to the 8 XCDs in turn
      * (id mod 8); with the pair count a multiple of 4, XCDs 0-3 take kv
      * head 0 and XCDs 4-7 kv head 1, so each XCD's L2 holds one head's K /
-     * V workspaces (4 MB at 4096 tokens) instead of both */
-    const int np = (p.nqb + 1) / 2, L = blockIdx.x;
+     * V workspaces (4 MB at 4096 tokens) instead of both.  SPLIT: the same
+     * over (q block, span) */
+    const int np = SPLIT ? p.nqb * p.spans : (p.nqb + 1) / 2, L = blockIdx.x;
     int x, g;
     if (p.kv_heads == 2 && (np & 3) == 0) {
         g = (L & 7) >> 2;
@@ -522,14 +530,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kern
     __shared__ __align__(16) _Float16 smem[4 * STAGE];   /* [group][stage] */
     __shared__ float sml[4][2][64];                      /* group B's m, l */
 
-    const int qL = p.nqb - 1 - x, qS = x;
-    const bool has_short = qS < qL;
-    const int nL = (min(p.t0 + 16 * qL + 16, end) + 31) >> 5;
+    /* SPLIT: one q block, tiles [c0, c0 + nL) of it; no short block.  The
+     * last block has the most tiles, and with them every span */
+    const int qL = p.nqb - 1 - (SPLIT ? x / p.spans : x), qS = x;
+    const bool has_short = !SPLIT && qS < qL;
+    const int nT = (min(p.t0 + 16 * qL + 16, end) + 31) >> 5;
+    const int c0 = SPLIT ? x % p.spans * p.span_tiles : 0;
+    if (SPLIT && c0 >= nT) return;              /* workgroup-uniform */
+    const int nL = SPLIT ? min(p.span_tiles, nT - c0) : nT;
     const int nS = has_short ? (min(p.t0 + 16 * qS + 16, end) + 31) >> 5 : 0;
     const int nA = (nL + nS + 1) >> 1;          /* intervals, and group A's tiles */
     const int nB = nS + nL - nA;                /* group B's tiles, nB <= nA */
     /* group B's j-th tile and its q block */
-    auto tile_b = [&](int j) { return j < nS ? j : nA + j - nS; };
+    auto tile_b = [&](int j) { return j < nS ? j : c0 + nA + j - nS; };
     auto block_b = [&](int j) { return j < nS ? qS : qL; };
 
     /* direct-to-LDS staging: this wave copies 1 KB blocks wg + 4i of a
@@ -695,17 +708,17 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kern
     const Dma2 dnone = dma2(0, 0, 0, 0, 0, 0);
     if (grp == 0) {
         load_q(p, g, qL, hl, col, h, qop);
-        stage_part(0, 0, 0);
-        stage_part(0, 1, 0);
+        stage_part(0, 0, c0);
+        stage_part(0, 1, c0);
         wait_dma();
         q35_lds_barrier();
         for (int it = 0; it < nA; it++) {
             /* the next tile's K and V, issued among this tile's QK MFMAs;
              * in the last interval the clamp reloads tile it into the
              * stage nobody reads again */
-            const int tn = min(it + 1, nA - 1);
+            const int tn = c0 + min(it + 1, nA - 1);
             qk(DmaOn<true>{}, dma2((it + 1) & 1, 0, tn, (it + 1) & 1, 1, tn), it & 1, s);
-            softmax_pv(DmaOn<false>{}, dnone, it & 1, s, it, qL);
+            softmax_pv(DmaOn<false>{}, dnone, it & 1, s, c0 + it, qL);
             wait_dma();
             q35_lds_barrier();
         }
@@ -772,14 +785,164 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kern
     if (grp == 0) {
         const float mB = sml[wg][0][lane], lB = sml[wg][1][lane];
         const float M = fmaxf(m_used, mB);
-        const float fa = exp2f_fast((m_used - M) * EXP_K);
+        /* (a later span can lie wholly after a column's position) */
+        const float fa = SPLIT && m_used == -INFINITY ? 0.0f : exp2f_fast((m_used - M) * EXP_K);
         const float fb = mB == -INFINITY ? 0.0f : exp2f_fast((mB - M) * EXP_K);
 #pragma unroll
         for (int dt = 0; dt < 8; dt++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[dt][i] = acc[dt][i] * fa + mrg[(16 * dt + i) * 64] * fb;
+        if (SPLIT && nL < nT) {
+            /* the span's partial, in register order: 1 KB a store */
+            const size_t slot = ((size_t)g * p.nqb + qL) * p.spans + x % p.spans;
+            float4 *po = reinterpret_cast<float4 *>(p.part) + (slot * 4 + wg) * 32 * 64 + lane;
+            float2 *pm = reinterpret_cast<float2 *>(p.part_ml) + (slot * 4 + wg) * 64 + lane;
+            *pm = make_float2(M, l_run * fa + lB * fb);
+#pragma unroll
+            for (int i = 0; i < 32; i++)
+                po[i * 64] = make_float4(acc[i >> 2][4 * (i & 3)], acc[i >> 2][4 * (i & 3) + 1],
+                                         acc[i >> 2][4 * (i & 3) + 2], acc[i >> 2][4 * (i & 3) + 3]);
+            return;
+        }
         store_rows(p, g, qL, hl, col, h, l_run * fa + lB * fb, acc);
     }
+}
+
+/* The spans of a q block added.  Workgroup (q block, wave wg of its four,
+ * pair u of the 32 float4 register groups): wave w takes spans w, w + 4, ...
+ * of wg's 32 columns, eight at a time with every load of a batch ahead of the
+ * first use, the four waves' (max, sum, O) meet in LDS in wave order, and
+ * wave 0 does the row store's O / l times sigmoid(gate).  Blocks of one span
+ * have stored their rows themselves.  One wave a (wg, pair) walking all spans
+ * was a chain of memory round trips: 16.7 us for 32 spans of 64 tokens. */
+constexpr int MERGE_U = 2, MERGE_SPLIT = 4 * 32 / MERGE_U, MERGE_BATCH = 8;
+__global__ __launch_bounds__(256) void span_merge_kernel(Q35GqaPrefill p) {
+    const int u = blockIdx.x & 15, wg = (blockIdx.x >> 4) & 3, unit = blockIdx.x / MERGE_SPLIT;
+    const int g = unit / p.nqb, qb = unit % p.nqb;
+    const int end = p.t0 + p.B;
+    const int nT = (min(p.t0 + 16 * qb + 16, end) + 31) >> 5;
+    const int n = (nT + p.span_tiles - 1) / p.span_tiles;
+    if (n < 2) return;                          /* workgroup-uniform */
+    const int lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const size_t slot = ((size_t)g * p.nqb + qb) * p.spans;
+    const float4 *po = reinterpret_cast<const float4 *>(p.part) + ((slot * 4 + wg) * 32 + MERGE_U * u) * 64 + lane;
+    const float2 *pm = reinterpret_cast<const float2 *>(p.part_ml) + (slot * 4 + wg) * 64 + lane;
+    float M = -INFINITY, L = 0.0f;
+    float o[MERGE_U][4] = {};
+    for (int c0 = w; c0 < n; c0 += 4 * MERGE_BATCH) {
+        float2 ml[MERGE_BATCH];
+        float4 a[MERGE_BATCH][MERGE_U];
+#pragma unroll
+        for (int k = 0; k < MERGE_BATCH; k++) {
+            const int c = c0 + 4 * k;
+            if (c >= n) {                       /* wave-uniform */
+                ml[k] = make_float2(-INFINITY, 0.0f);
+#pragma unroll
+                for (int v = 0; v < MERGE_U; v++) a[k][v] = make_float4(0.f, 0.f, 0.f, 0.f);
+                continue;
+            }
+            ml[k] = pm[c * 4 * 64];
+#pragma unroll
+            for (int v = 0; v < MERGE_U; v++) a[k][v] = po[(size_t)c * 4 * 32 * 64 + v * 64];
+        }
+        float mx = M;
+#pragma unroll
+        for (int k = 0; k < MERGE_BATCH; k++) mx = fmaxf(mx, ml[k].x);
+        /* spans wholly after a column's position carry -inf, 0, 0 */
+        const float mk = mx == -INFINITY ? 0.0f : mx;
+        const float fo = exp2f_fast((M - mk) * EXP_K);
+        L *= fo;
+#pragma unroll
+        for (int v = 0; v < MERGE_U; v++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[v][e] *= fo;
+#pragma unroll
+        for (int k = 0; k < MERGE_BATCH; k++) {
+            const float f = exp2f_fast((ml[k].x - mk) * EXP_K);
+            L += ml[k].y * f;
+#pragma unroll
+            for (int v = 0; v < MERGE_U; v++) {
+                o[v][0] += a[k][v].x * f;
+                o[v][1] += a[k][v].y * f;
+                o[v][2] += a[k][v].z * f;
+                o[v][3] += a[k][v].w * f;
+            }
+        }
+        M = mx;
+    }
+    __shared__ float sm[4][2 + 4 * MERGE_U][64];
+    sm[w][0][lane] = M;
+    sm[w][1][lane] = L;
+#pragma unroll
+    for (int i = 0; i < 4 * MERGE_U; i++) sm[w][2 + i][lane] = o[i >> 2][i & 3];
+    q35_lds_barrier();
+    if (w != 0) return;
+    /* the largest max is finite: span 0, which wave 0 merged, holds key 0 */
+    float mx = M;
+#pragma unroll
+    for (int i = 1; i < 4; i++) mx = fmaxf(mx, sm[i][0][lane]);
+    const float f0 = exp2f_fast((M - mx) * EXP_K);
+    L *= f0;
+#pragma unroll
+    for (int i = 0; i < 4 * MERGE_U; i++) o[i >> 2][i & 3] *= f0;
+#pragma unroll
+    for (int k = 1; k < 4; k++) {
+        const float f = exp2f_fast((sm[k][0][lane] - mx) * EXP_K);
+        L += sm[k][1][lane] * f;
+#pragma unroll
+        for (int i = 0; i < 4 * MERGE_U; i++) o[i >> 2][i & 3] += sm[k][2 + i][lane] * f;
+    }
+    L += __shfl_xor(L, 32);
+    const int b = 16 * qb + (col & 15), head = g * G + 2 * wg + (col >> 4);
+    if (b >= p.B) return;
+    const float inv = 1.0f / L;
+    const size_t row = (size_t)b * p.heads + head;
+#pragma unroll
+    for (int v = 0; v < MERGE_U; v++) {
+        const int i = MERGE_U * u + v, d = 32 * (i >> 2) + 8 * (i & 3) + 4 * h;
+        const float4 gv = *reinterpret_cast<const float4 *>(p.q_gate + row * 2 * D + D + d);
+        *reinterpret_cast<float4 *>(p.attn_out + row * D + d) =
+            make_float4(o[v][0] * inv * q35_sigmoid_fast(gv.x), o[v][1] * inv * q35_sigmoid_fast(gv.y),
+                        o[v][2] * inv * q35_sigmoid_fast(gv.z), o[v][3] * inv * q35_sigmoid_fast(gv.w));
+    }
+}
+
+/* Spans of a q block's tiles, or 0 for the pair form, by the smaller of the
+ * two forms' costs in intervals (one tile a group, 1.3 us on a nearly idle
+ * GPU, 2.3 with a workgroup on every CU) on 256 CUs, one workgroup each:
+ *   - a workgroup's start and end (q's norm and rotation, the first tiles,
+ *     the merge of its groups, the rows) are 6; the pair form does them for
+ *     its two blocks in turn, 10 more;
+ *   - partials cost 1 for the merge launch and 0.07 a span for the 256 KB
+ *     its two kv heads write and read (so spans of a few tiles lose: 64
+ *     tokens at 4032 in 8 / 16 / 32 spans 40.9 / 36.7 / 39.1 us, whole op);
+ *   - past 256 workgroups, blocks go longest first: the end is the average
+ *     load, half of the shortest block and 14 for the uneven last round.
+ * The pair form is left for more than 128 blocks that start near position
+ * 0, whose lengths differ most (at 0, pairs / one span a block: 4096 tokens
+ * 184 / 191 us, 3500 132 / 137; but 2048 90 / 79, 64 32.3 / 26.8, 5000 335 /
+ * 275, whose pairs need a second round; 2500 at 2000 191 / 186).  The
+ * 500-token prefill at 12345 took 582 us with pairs (32 workgroups) and 131
+ * in 4 spans, 64 tokens at 32000 1318 and 79 in 32. */
+constexpr int CUS = 256;
+int spans_for(int t0, int B, int *span_tiles) {
+    const int nqb = (B + 15) / 16, n1 = (min(t0 + 16, t0 + B) + 31) / 32, n2 = (t0 + B + 31) / 32;
+    double best = ((nqb + 1) / 2 * 2 + CUS - 1) / CUS * ((n1 + n2 + 1) / 2 + 16.0);
+    int spans = 0;
+    *span_tiles = n2;
+    for (int S = 1; S <= n2 && (S == 1 || 2 * nqb * S <= CUS); S++) {
+        const int tiles = (n2 + S - 1) / S;
+        double cost = 6 + (tiles + 1) / 2;
+        if (S > 1) cost += 1 + 0.07 * nqb * S;
+        else if (2 * nqb > CUS) cost = (6 + 0.25 * (n1 + n2)) * 2 * nqb / CUS + 14 + 0.25 * n1;
+        if (cost < best) {
+            best = cost;
+            spans = (n2 + tiles - 1) / tiles;
+            *span_tiles = tiles;
+        }
+    }
+    return spans;
 }
 
 }  // namespace
@@ -788,6 +951,11 @@ extern "C" void q35_gqa_prefill_ws_bytes(int t0, int B, int kv_heads, size_t *kw
     const size_t kbt = (size_t)(t0 + B + 31) / 32;
     *kw = (size_t)kv_heads * kbt * 32 * D * 2;
     *vw = *kw;
+}
+
+extern "C" size_t q35_gqa_prefill_part_bytes(size_t *ml) {
+    *ml = (size_t)CUS * 128 * 2 * 8;
+    return (size_t)CUS * 128 * D * 4;
 }
 
 extern "C" hipError_t q35_gqa_prefill(const Q35GqaPrefill *pin, hipStream_t stream) {
@@ -805,6 +973,14 @@ extern "C" hipError_t q35_gqa_prefill(const Q35GqaPrefill *pin, hipStream_t stre
     hipLaunchKernelGGL(prep_kernel, dim3((unsigned)nblk), dim3(256), 0, stream, p, nvb, n_rows);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(attn_kernel, dim3((p.nqb + 1) / 2 * p.kv_heads), dim3(512), 0, stream, p);
+    p.spans = spans_for(p.t0, p.B, &p.span_tiles);
+    if (p.spans == 0) {
+        hipLaunchKernelGGL(attn_kernel<false>, dim3((p.nqb + 1) / 2 * p.kv_heads), dim3(512), 0, stream, p);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(attn_kernel<true>, dim3(p.nqb * p.spans * p.kv_heads), dim3(512), 0, stream, p);
+    e = hipGetLastError();
+    if (e != hipSuccess || p.spans == 1) return e;
+    hipLaunchKernelGGL(span_merge_kernel, dim3(p.nqb * p.kv_heads * MERGE_SPLIT), dim3(256), 0, stream, p);
     return hipGetLastError();
 }

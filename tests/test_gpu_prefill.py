@@ -257,6 +257,40 @@ def test_gqa_prefill_unaligned_start(t0, B):
         ga.close()
 
 
+@pytest.mark.parametrize("t0,B", [(31, 2), (300, 23), (991, 37), (1000, 16), (2047, 33), (3001, 130), (6000, 1)])
+def test_gqa_prefill_spans(t0, B):
+    """Short chunks over a longer cache, whose q blocks run as spans of key
+    tiles and a merge: one span and many, a last span of one tile that lies
+    wholly after its block's first positions, batch remainders, one token.
+    Against float64 over the drawn bf16 cache.  The operands are fp16 (2^-11
+    relative): outputs average values of about 1, and ATOL is the bar of
+    every test here."""
+    from ds4f_hip.lib import check, load
+    import f64_model as F
+
+    _say(f"gqa prefill spans t0={t0} B={B}")
+    cache = KvCache(1, t0 + B + 8)
+    ga = GpuAttention([2], t0 + B + 8, cache)
+    try:
+        check(load().ds4f_hip_synth_gqa_cache(0, t0, 0, S.tid(S.GQA_KCACHE, 0),
+                                              S.tid(S.GQA_VCACHE, 0), None), "synth kv")
+        ga.sync(0, to_host=True, n_kv_tokens=t0)
+        half = GQ.kv_heads * GQ.head_dim
+        past = cache.kv[0, :t0].astype(np.float64)
+        shape = (t0, GQ.kv_heads, GQ.head_dim)
+        qn, kn = W.gqa_weights(GQ)
+        q, k, v = W.gqa_prefill_tokens(GQ, B)
+        out, _ = ga.gqa_prefill(0, t0, q.reshape(B, -1), k.reshape(B, -1), v.reshape(B, -1), qn, kn)
+        ref, _ = F.gqa_prefill(q, k, v, qn, kn, t0, past[:, :half].reshape(shape),
+                               past[:, half:].reshape(shape))
+        mx, rr = _err(out.reshape(-1), ref.reshape(-1))
+        _say(f"  max abs {mx:.3e} rel-rms {rr:.3e}")
+        assert np.isfinite(out).all()
+        assert mx <= ATOL
+    finally:
+        ga.close()
+
+
 # ------------------------------------------------------------------ delta rule
 LG = W.LinGeom()
 STATE_RTOL = 1e-4
