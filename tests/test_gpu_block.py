@@ -242,6 +242,10 @@ def _chunk_passes(T, n_pass, graph):
         def launch():
             stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
             states.copy_(states0)
+            if not torch.cuda.is_current_stream_capturing():
+                # torch's default stream is the null handle, for which the plugin takes
+                # its own non-blocking stream: nothing orders that behind the copy
+                torch.cuda.current_stream().synchronize()
             for Lr in range(2):
                 rc = ga.lib.ds4f_hip_attn_chunk_async(Lr, 0, T, dptr(states), stream)
                 assert rc == 0, ga.lib.ds4f_gpu_last_error()
