@@ -1231,7 +1231,7 @@ int ds4f_gpu_attn_weights(int L, const Ds4fGpuLayerW *w) {
     int n = 0;
     for (int i = 0; i < np; i++) n += mlx4_parts(pt + n, proj[i], &pv[i], &ps[i], &pb[i]);
     n += mlx4_parts(pt + n, outw, &pv[4], &ps[4], &pb[4]);
-    /* (16 s, b - 16 s) per row and 64-column group of each weight, for the
+    /* the scale and bias per row and 64-column group of each weight, for the
      * chunk GEMMs (filled on the device below) */
     for (int i = 0; i < 5; i++) {
         const Ds4fGpuMlx4W *m = i < 4 ? (i < np ? proj[i] : NULL) : outw;
@@ -1388,7 +1388,7 @@ int ds4f_gpu_attn_step(int L, int token, float *state) {
 /* ---- whole-layer chunks (ds4f_attn_gqa_chunk :1145-1252,
  * ds4f_attn_linear_chunk :977-1135) ------------------------------------- */
 
-/* chunk workspace of mpad token rows: X operands (hi, lo, group sums) for
+/* chunk workspace of mpad token rows: X operands (digits, group sums) for
  * K up to 4096, the projection outputs of either layer kind, the core's
  * output; grow-only */
 enum { CH_Q, CH_K, CH_V, CH_AO, CH_QKV, CH_Z, CH_A, CH_B, CH_LO, CH_N };
@@ -1418,7 +1418,7 @@ typedef struct { uint16_t *xw; float *xsum; float *out[CH_N]; } ChunkWs;
 static size_t chunk_layout(int mpad, ChunkWs *ws) {
     const size_t K = ch_kmax();
     size_t sizes[2 + CH_N], off[2 + CH_N], total = 0;
-    sizes[0] = (size_t)mpad * K * 4;            /* fp16 hi and lo */
+    sizes[0] = (size_t)mpad * K * 4;            /* the X digits */
     sizes[1] = (K / 64) * (size_t)mpad * 4;
     for (int i = 0; i < CH_N; i++) sizes[2 + i] = (size_t)mpad * ch_width(i) * 4;
     for (int i = 0; i < 2 + CH_N; i++) {

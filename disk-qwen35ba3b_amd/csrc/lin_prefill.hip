@@ -765,22 +765,26 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_kernel(Q35LinPrefill p) {
     }
 }
 
-/* ---- 5. RMSNormGated per (4 tokens, value head), in place on out ------- *
- * grid (VH / 4, ceil(B / GTT)), wave w -> head 4*blockIdx.x + w of GTT
+/* ---- 5. RMSNormGated per (TT tokens, value head) ----------------------- *
+ * grid (VH / 4, ceil(B / TT)), wave w -> head 4*blockIdx.x + w of TT
  * consecutive tokens, 2 columns a lane.  Every token's o and z rows are
- * requested before the first is used (GTT = 4 against one token a wave:
+ * requested before the first is used (4 tokens a wave against one:
  * 35.7 -> 30.9 us at 4096 tokens, the kernel then at the HBM copy rate).
  * The reference's operation order (src/attn_qwen.c:726-749) with an fp32
  * square sum, x times 1 / r and the sigmoid on v_exp / v_rcp (about 1 ulp
- * each; the prefill outputs are checked to 2e-3). */
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-
+ * each; the prefill outputs are checked to 2e-3).
+ * XW false: in place on out.  XW true: the chunk GEMM's X operand instead.
+ * A lane of that operand is 32 columns of a row, so the wave's rows pass
+ * through its own LDS area and lane (token l % TT, quarter l / TT of the
+ * head) stores the digits, 16 TT consecutive bytes a quarter. */
 constexpr int GTT = 4;
-template <int TT>
+template <int TT, bool XW>
 __global__ __launch_bounds__(256) void gnorm_kernel(Q35LinPrefill p) {
-    const int h = 4 * blockIdx.x + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int b0 = blockIdx.y * TT;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int h = 4 * blockIdx.x + w, b0 = blockIdx.y * TT;
     const uint32_t nw = *reinterpret_cast<const uint32_t *>(p.norm_w + 2 * lane);
+    constexpr int RS = VD + 4;      /* row stride: 16 rows' 16-byte reads on distinct banks */
+    __shared__ __align__(16) float rows[XW ? 4 : 1][XW ? TT * RS : 4];
     float2 oa[TT], za[TT];
 #pragma unroll
     for (int k = 0; k < TT; k++) {
@@ -789,61 +793,54 @@ __global__ __launch_bounds__(256) void gnorm_kernel(Q35LinPrefill p) {
         oa[k] = *reinterpret_cast<const float2 *>(p.out + off);
         za[k] = *reinterpret_cast<const float2 *>(p.z + off);
     }
-    float2 y[TT];
 #pragma unroll
     for (int k = 0; k < TT; k++) {
         const float2 o = oa[k], z = za[k];
         float ss = o.x * o.x + o.y * o.y;
         ss = q35_wave_sum(ss);
+        float2 y;
         {
 #pragma clang fp contract(off)
             const float r = sqrtf(ss * (1.0f / (float)VD) + 1e-6f), ri = 1.0f / r;
-            y[k].x = o.x * ri * q35_bf2f((uint16_t)(nw & 0xffff)) * (z.x * q35_sigmoid_fast(z.x));
-            y[k].y = o.y * ri * q35_bf2f((uint16_t)(nw >> 16)) * (z.y * q35_sigmoid_fast(z.y));
+            y.x = o.x * ri * q35_bf2f((uint16_t)(nw & 0xffff)) * (z.x * q35_sigmoid_fast(z.x));
+            y.y = o.y * ri * q35_bf2f((uint16_t)(nw >> 16)) * (z.y * q35_sigmoid_fast(z.y));
         }
-        if (!p.xw && b0 + k < p.B)
-            *reinterpret_cast<float2 *>(p.out + ((size_t)(b0 + k) * p.v_heads + h) * VD + 2 * lane) = y[k];
+        if constexpr (XW)
+            *reinterpret_cast<float2 *>(&rows[w][k * RS + 2 * lane]) = y;
+        else if (b0 + k < p.B)
+            *reinterpret_cast<float2 *>(p.out + ((size_t)(b0 + k) * p.v_heads + h) * VD + 2 * lane) = y;
     }
-    if (!p.xw) return;
-    /* The chunk GEMM's X operand instead: quad lanes 4w..4w+3 hold word w of
-     * the head's 16 (values 2i, 2i + 1 in quad lane i) of every token; quad
-     * lane i gathers token b0 + i's word and stores its granules, so the quad
-     * writes 64 consecutive bytes (the tokens are consecutive operand rows).
-     * The group sums (64 columns = one half wave) add the same hi + lo. */
-    static_assert(TT == 4, "one token a quad lane");
-    const int G = p.v_heads * VD / 64, v = h * (VD / 8) + (lane >> 2), qi = lane & 3;
-    float w8[8];
-    bool over = false;
+    if constexpr (XW) {
+        const int k = lane % TT, quarter = lane / TT, b = b0 + k;
+        if (quarter >= 4) return;
+        f32x16_t v[2];
+        float s = 0.0f, mx = 0.0f;
 #pragma unroll
-    for (int k = 0; k < TT; k++) {
-        over = over || q35_f16_over(y[k].x) || q35_f16_over(y[k].y);
-        const float g8[8] = {q35_dpp<0x00>(y[k].x), q35_dpp<0x00>(y[k].y), q35_dpp<0x55>(y[k].x),
-                             q35_dpp<0x55>(y[k].y), q35_dpp<0xAA>(y[k].x), q35_dpp<0xAA>(y[k].y),
-                             q35_dpp<0xFF>(y[k].x), q35_dpp<0xFF>(y[k].y)};
+        for (int i = 0; i < 8; i++) {
+            const float4 x = *reinterpret_cast<const float4 *>(&rows[w][k * RS + 32 * quarter + 4 * i]);
 #pragma unroll
-        for (int j = 0; j < 8; j++) w8[j] = k == 0 || qi == k ? g8[j] : w8[j];
-        const _Float16 hx = (_Float16)y[k].x, hy = (_Float16)y[k].y;
-        float s = ((float)hx + (float)(_Float16)(y[k].x - (float)hx)) +
-                  ((float)hy + (float)(_Float16)(y[k].y - (float)hy));
-        s = q35_half_sum(s);
-        if ((lane & 31) == 0 && b0 + k < p.B) p.xsum[(size_t)(v >> 3) * p.mpad + b0 + k] = s;
-    }
-    /* (tokens past the batch repeat its last row: no new value to check) */
-    q35_f16_guard(p.status, Q35_STATUS_GEMM_F16, over);
-    f16x8 hi, lo;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const float x = w8[q35_xw_perm(j)];
-        hi[j] = (_Float16)x;
-        lo[j] = (_Float16)(x - (float)hi[j]);
-    }
-    if (b0 + qi < p.B) {
-        uint8_t *gr = reinterpret_cast<uint8_t *>(p.xw) + q35_xw_granule(b0 + qi, v, G);
-        *reinterpret_cast<f16x8 *>(gr) = hi;
-        *reinterpret_cast<f16x8 *>(gr + Q35_XW_BLK) = lo;
+            for (int e = 0; e < 4; e++) {
+                v[i >> 2][4 * (i & 3) + e] = el(x, e);
+                s += el(x, e);
+                mx = fmaxf(mx, fabsf(el(x, e)));
+            }
+        }
+        /* (tokens past the batch repeat its last row: no new value to check) */
+        q35_f16_guard(p.status, Q35_STATUS_GEMM_F16, q35_f16_over(mx));
+        const float s2 = s + __shfl_xor(s, TT);
+        if (b >= p.B) return;
+        const int G = p.v_heads * VD / 64, g = h * (VD / 64) + (quarter >> 1), half = quarter & 1;
+        q35_xw_store(reinterpret_cast<uint8_t *>(p.xw) + q35_xw_block(b, g, G), 32 * half + (b & 31), v[0], v[1],
+                     s, mx);
+        if (half == 0) p.xsum[(size_t)g * p.mpad + b] = s2;
     }
 }
 
+template <int TT, bool XW>
+hipError_t launch_gnorm(const Q35LinPrefill &p, hipStream_t stream) {
+    hipLaunchKernelGGL((gnorm_kernel<TT, XW>), dim3(p.v_heads / 4, (p.B + TT - 1) / TT), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
 
 }  // namespace
 
@@ -874,8 +871,9 @@ extern "C" hipError_t q35_lin_prefill(const Q35LinPrefill *pin, hipStream_t stre
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(scan_kernel, dim3(p.v_heads * (VD / 16)), dim3(SCAN_THREADS), 0, stream, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(gnorm_kernel<GTT>, dim3(p.v_heads / 4, (p.B + GTT - 1) / GTT), dim3(256), 0, stream, p);
-    return hipGetLastError();
+    if (!p.xw) return launch_gnorm<GTT, false>(p, stream);
+    /* 16 tokens a wave convert on all 64 lanes; short chunks take more, smaller workgroups */
+    return p.B <= 512 ? launch_gnorm<4, true>(p, stream) : launch_gnorm<16, true>(p, stream);
 }
 
 /* ---- the workspace of the no-allocation entry point ---------------------

@@ -7,197 +7,173 @@
  *
  * Exactness.  With w = q s + b (q in 0..15, s and b the BF16 scale and
  * bias of the 64-element group), and G the groups along K,
- *     y[m][n] = sum_g s'[n,g] sum_{k in g} (1 + q/16) x  +  b'[n,g] xsum[m,g],
- *     s' = 16 s,  b' = b - 16 s,  xsum[m,g] = sum_{k in g} x.
- * 1 + q/16 is exact in fp16 (the nibble in mantissa bits 6..9 under the
- * exponent of 1), x is carried as an fp16 hi + lo pair (about 22 bits),
- * each MFMA product is exact in fp32, and the group partial is scaled by
- * s' in fp32 after its 8 MFMAs (4 k-steps x hi / lo); xsum is the sum of
- * the same hi + lo values.  The offset 1 is at most about twice the q/16
- * part, so the cancellation against b' xsum costs about a bit, and the
- * result differs from the reference's fp32 dot products by fp32 rounding
- * of the group sums.
+ *     y[m][n] = sum_g s[n,g] sum_{k in g} q x  +  sum_g b[n,g] xsum[m,g],
+ *     xsum[m,g] = sum_{k in g} x.
+ * Both operands of the group product are fp6 (e2m3): the nibble q zero-
+ * extended to six bits is the code of q / 8, and x is five fp6 digits under
+ * per-32-column exponents (q35_xw_store, 2^-24 of the columns' largest
+ * value), each an operand of v_mfma_scale_f32_32x32x64_f8f6f4.  A product
+ * of two digits is exact, a group's five digits are added from the lowest
+ * up in one fp32 accumulator, and the group sum is scaled by s in fp32.  The
+ * bias term is a product of its own over the groups: b is BF16 and xsum
+ * three BF16 parts (24 bits), exact products added in fp32.
+ * MFMA cycles per 32 x 32 outputs and group: 5 x 32; as fp16 (x as hi + lo, 22
+ * bits) they were 8 x 32.
  *
  * Layouts:
- *   xw      (xprep_kernel) per 64-token tile mt and group g, a 16 KB block
- *           at ((mt G + g) 2 + {0: hi, 1: lo}) 8 KB, fp16: the group's MFMA
- *           operands as the waves read them, 1 KB each (q35_xw_granule); 8
- *           consecutive k (one nibble word's worth) kept in the order
- *           0,4,1,5,2,6,3,7, the order in which a word's nibbles become fp16
- *           pairs (nibbles j and j + 4 moved to bits 6..9 and 22..25, ORed
- *           into 0x3C003C00, give 1 + q_j / 16 and 1 + q_{j+4} / 16);
+ *   xw      (xprep_kernel) the X digits in operand order (q35_device.h);
  *   xsum    fp32 [G][Mpad];
- *   sb      (sb_kernel) (16 s, b - 16 s) as [G][Npad], Npad = N rounded up
- *           to 256, zeros past N;
- *   wt      (wt_kernel) the weight words re-laid out once per weight: per
- *           256-feature tile and group an 8 KB block that is the LDS image
- *           of the stage (16-byte position p = row p / 2, half
- *           wslot(row, p % 2)), rows past N zero; staging it is a plain
- *           copy, 1 KB a wave load.
- * In a group (8 words), MFMA k-step ks of lane half h is word 4h + ks: a
- * lane's weight operand for a whole group is one 16-byte read.
+ *   sb      (sb_kernel) s as fp32 [G][Npad], then b as BF16 [G][Npad],
+ *           Npad = N rounded up to 256, zeros past N;
+ *   wt      (wt_kernel) the nibbles re-laid out once per weight: per
+ *           256-row tile and group, a block of 256 rows x 32 bytes, the
+ *           16 bytes of half h (columns 32h .. of the group) of row r at slot
+ *           wslot(r, h) of the row.  A lane's 32 nibbles become its
+ *           operand's 192 bits with 8 instructions (expand_fp6).
  *
- * gemm_kernel: 256 threads, a 64-token x 256-feature tile; wave w owns
- * features 64w..64w+63 as 2 x 2 blocks of v_mfma_f32_32x32x16_f16 (A = X,
- * B = W^T converted in registers).  Every global load is a direct-to-LDS
- * load into a ring of three stages, one group each (X hi and lo 16 KB,
- * the tile's weight words 8 KB, (s, b') 2 KB, xsum 256 B), issued two
- * groups ahead (every stage load a contiguous 1 KB); each wave waits for
- * its own loads of the next group
- * before the one barrier a group.  Two workgroups fit a CU (157.5 KB of
- * LDS), two waves a SIMD.
+ * gemm_kernel: a 64-token x 256-feature tile, 4 waves; a wave owns 32
+ * tokens x 128 features as four 32 x 32 blocks (A = X, B = W^T).  Every
+ * global load is a direct-to-LDS load into a ring of three stages, one
+ * group each (X 16 KB, the nibbles 8 KB, s 1 KB), issued two and a half groups
+ * ahead, every stage load a contiguous 1 KB.  A wave reads its X of group
+ * g + 1 into registers under the MFMAs of group g and scales a pair of blocks
+ * under the next pair's MFMAs, so the MFMAs wait neither for LDS after the one
+ * barrier a group nor for the fp32 work.  The bias term starts the
+ * accumulators, while the first stages arrive.  Two workgroups fit a CU, so
+ * one's start and stores run under the other's MFMAs.
+ * What bounds it: at 4096 tokens the MFMA pipes are busy 46 % of the time at
+ * 1.9 GHz (the rate of this instruction alone with random operands is power-
+ * limited, 24 ns an MFMA against 13 nominal); without the stage loads 96 ->
+ * 81 us a 2048 x 4096 product, with a fifth of the MFMAs 55.  us a launch at
+ * 4096 tokens, x as fp16 hi + lo -> here: projections 12352 x 2048 383 -> 290,
+ * 9216 x 2048 275 -> 208, output 2048 x 4096 115 -> 94.  512 features a
+ * workgroup (8 waves, a third less staging) 312, 227 and 90.
  * gemm_few_kernel: the same product split over K inside a workgroup, for
  * chunks of few tokens (few_tokens picks).
  */
 #include "q35_device.h"
 #include "q35_launch.h"
 
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+typedef __attribute__((ext_vector_type(8))) int i32x8_t;
 
 namespace {
 
-constexpr int NT = 256;
 constexpr int MT = 64;                 /* tokens a tile */
-constexpr int NTILE = 256;             /* features a tile, 64 a wave */
-constexpr int XBLK = Q35_XW_BLK;       /* bytes of a tile's hi (or lo) X of one group */
-static_assert(MT == Q35_XW_ROWS, "the X tiles are the GEMM's token tiles");
-constexpr int WBLK = NTILE * 32;       /* bytes of a tile's weight words of one group */
-constexpr int SBLK = NTILE * 8;        /* bytes of a tile's (s, b') of one group */
-constexpr int OFF_W = 2 * XBLK, OFF_SB = OFF_W + WBLK, OFF_XS = OFF_SB + SBLK;
-constexpr int STAGE = OFF_XS + MT * 4; /* 26880 bytes */
-constexpr int NSTAGE = 3;
-constexpr float QSTEP = 16.0f;         /* B = 1 + q / QSTEP */
+constexpr int NTILE = 256;             /* features of a weight tile */
+static_assert(MT == Q35_XW_ROWS, "X is allocated in the GEMM's token tiles");
+constexpr int XBLK = Q35_XW_BLK;
+constexpr int WBLK = NTILE * 32;       /* bytes of a weight tile's nibbles of one group */
 
-/* slot of half h (words 4h..4h+3) of tile feature row r in its 32-byte
+/* slot of half h (columns 32h .. of a group) of tile feature row r in its 32-byte
  * weight row: distinct over 4 and 8 consecutive rows, so the operand reads are
  * free of bank conflicts */
 __device__ __forceinline__ int wslot(int r, int h) { return h ^ (((r >> 2) ^ (r >> 3)) & 1); }
 
-/* x rows -> (optional RMSNorm) -> fp16 hi / lo operands and the group sums of
- * hi + lo.  One workgroup of NTX threads per XR token rows: thread t holds
- * row t % XR, words t / XR + i NTX / XR (WT of them), so the lanes of a
- * 64-column group are 8 XR neighbours, reads are 256 consecutive bytes of each
- * row and stores 16 XR bytes of the operand image.  XR = 8 stores whole
- * 128-byte lines, but with few tokens it is few workgroups that convert 8
- * rows each; launch_xprep has the line.
- * Rows at and past M in the last workgroup are stored as zeros; operand rows
- * after those are never written: an operand row only reaches its own output
- * row, which is not stored.  The norm is an fp32 square sum times the hardware
- * rsq (about 1 ulp from the reference's double sum and division,
- * src/attn_qwen.c:142-157, far below the hi / lo split's 22 bits). */
-/* sum over the 8 lanes of one row's words of a group (8 XR neighbouring
- * lanes, equal lane % XR), the total in each of them */
-template <int XR>
-__device__ __forceinline__ float group_sum(float v) {
-    static_assert(XR == 8 || XR == 4 || XR == 2, "lane patterns of 2, 4 and 8 rows");
-    v += q35_xor8(v);
-    if constexpr (XR == 8) return q35_psum32(q35_psum16(v));
-    v += q35_dpp<0x124>(v);                /* row_ror:4, on sums of period 8 */
-    if constexpr (XR == 4) return q35_psum16(v);
-    return v + q35_dpp<0x122>(v);          /* row_ror:2, on sums of period 4 */
-}
-template <int NTX, int XR, int WT>
+/* x rows -> (optional RMSNorm) -> the X digits and the group sums.  One
+ * workgroup of NTX threads per XR token rows: thread t holds 32 consecutive
+ * columns 32 (t / XR) .. of row t % XR, so the two lanes of a 64-column group
+ * are XR apart and stores are 16 XR and 8 XR consecutive bytes of the operand
+ * image.  XR = 8 stores whole 128-byte lines, but with few tokens it is few
+ * workgroups that convert 8 rows each; q35_mlx4_xprep has the line.
+ * Operand rows at and past M are never written: an operand row only reaches
+ * its own output row, which is not stored.  The norm is an fp32 square sum
+ * times the hardware rsq (about 1 ulp from the reference's double sum and
+ * division, src/attn_qwen.c:142-157). */
+template <int NTX, int XR>
 __global__ __launch_bounds__(NTX) void xprep_kernel(Q35Mlx4Xprep p) {
-    const int t = threadIdx.x, lane = t & 63, r = t % XR;
+    const int t = threadIdx.x, lane = t & 63, r = t % XR, hg = t / XR;
     const int m0 = blockIdx.x * XR, m = m0 + r;
-    const int nw = p.K / 8;
+    const bool in = 32 * hg < p.K;           /* K is a multiple of 64: both lanes of a group */
     __shared__ float sred[NTX / 64][XR];
 
-    /* the thread's words of its row and of the norm weight, all requested
-     * at once as range-checked buffer loads (rows past M, words past K and
-     * an absent norm weight read as zeros): the norm and the conversion
-     * then work from registers, one memory round trip a workgroup */
+    /* the thread's columns of its row and of the norm weight, all requested
+     * at once as range-checked buffer loads (rows past M, columns past K and
+     * an absent norm weight read as zeros) */
     const int nr = min(XR, p.M - m0);
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<float *>(p.x + (size_t)m0 * p.ldx)), 0, ((nr - 1) * p.ldx + p.K) * 4,
         Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<uint16_t *>(p.norm_w)), 0, p.norm_w ? p.K * 2 : 0, Q35_BUF_DW3);
-    float4 xa[WT], xb[WT];
-    uint4 wv[WT];
+    const uint32_t off = in && r < nr ? (uint32_t)(r * p.ldx + 32 * hg) * 4 : 0x80000000u;
+    float4 x[8];
+    uint4 wv[4];
 #pragma unroll
-    for (int i = 0; i < WT; i++) {
-        const int v = t / XR + i * (NTX / XR);
-        const uint32_t off = v < nw && r < nr ? (uint32_t)(r * p.ldx + 8 * v) * 4 : 0x80000000u;
-        xa[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0));
-        xb[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off + 16, 0, 0));
-        wv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs, 16 * v, 0, 0));
+    for (int i = 0; i < 8; i++)
+        x[i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(xrs, off + 16 * i, 0, 0));
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        wv[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrs, 64 * hg + 16 * i, 0, 0));
+    f32x16_t v[2];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        v[i >> 2][4 * (i & 3)] = x[i].x;
+        v[i >> 2][4 * (i & 3) + 1] = x[i].y;
+        v[i >> 2][4 * (i & 3) + 2] = x[i].z;
+        v[i >> 2][4 * (i & 3) + 3] = x[i].w;
     }
 
-    float ri = 1.0f;
     if (p.norm_w) {
         float ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < WT; i++) {
-            const float e[8] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w, xb[i].x, xb[i].y, xb[i].z, xb[i].w};
+        for (int i = 0; i < 32; i++) ss = fmaf(v[i >> 4][i & 15], v[i >> 4][i & 15], ss);
 #pragma unroll
-            for (int j = 0; j < 8; j++) ss = fmaf(e[j], e[j], ss);
-        }
-        ss = group_sum<XR>(ss);
-        if constexpr (XR == 2) ss = q35_psum16(ss);
-        if constexpr (XR <= 4) ss = q35_psum32(ss);
+        for (int o = XR; o < 64; o <<= 1) ss += __shfl_xor(ss, o);
         if (lane < XR) sred[t >> 6][lane] = ss;
         q35_lds_barrier();
         ss = 0.0f;
 #pragma unroll
         for (int i = 0; i < NTX / 64; i++) ss += sred[i][r];
-        ri = __builtin_amdgcn_rsqf(ss * (1.0f / (float)p.K) + 1e-6f);
-    }
+        const float ri = __builtin_amdgcn_rsqf(ss * (1.0f / (float)p.K) + 1e-6f);
 #pragma unroll
-    for (int i = 0; i < WT; i++) {
-        const int v = t / XR + i * (NTX / XR);
-        if (v >= nw) break;   /* nw is a multiple of 8: a group's 8 words leave together */
-        float e[8] = {xa[i].x, xa[i].y, xa[i].z, xa[i].w, xb[i].x, xb[i].y, xb[i].z, xb[i].w};
-        if (p.norm_w) {
-            const uint32_t ww[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w};
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                e[j] = e[j] * ri * q35_bf2f((uint16_t)(ww[j >> 1] >> (16 * (j & 1))));
+        for (int i = 0; i < 32; i++) {
+            const uint32_t ww = (i & 6) == 0 ? wv[i >> 3].x : (i & 6) == 2 ? wv[i >> 3].y
+                                : (i & 6) == 4 ? wv[i >> 3].z : wv[i >> 3].w;
+            v[i >> 4][i & 15] = v[i >> 4][i & 15] * ri * q35_bf2f((uint16_t)(ww >> (16 * (i & 1))));
         }
-        bool over = false;
-#pragma unroll
-        for (int j = 0; j < 8; j++) over = over || q35_f16_over(e[j]);
-        q35_f16_guard(p.status, Q35_STATUS_GEMM_F16, over);
-        f16x8_t hi, lo;
-        float s = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float v8 = e[q35_xw_perm(j)];
-            const _Float16 h = (_Float16)v8;
-            const _Float16 l = (_Float16)(v8 - (float)h);
-            hi[j] = h;
-            lo[j] = l;
-            s += (float)h + (float)l;
-        }
-        uint8_t *blk = reinterpret_cast<uint8_t *>(p.xw) + q35_xw_granule(m, v, p.K / 64);
-        *reinterpret_cast<f16x8_t *>(blk) = hi;
-        *reinterpret_cast<f16x8_t *>(blk + XBLK) = lo;
-        s = group_sum<XR>(s);
-        if ((lane & (8 * XR - 1)) < XR) p.xsum[(size_t)(v >> 3) * p.Mpad + m] = s;
     }
+    float s = 0.0f, mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i++) {
+        s += v[i >> 4][i & 15];
+        mx = fmaxf(mx, fabsf(v[i >> 4][i & 15]));
+    }
+    q35_f16_guard(p.status, Q35_STATUS_GEMM_F16, in && q35_f16_over(mx));
+    const float s2 = s + __shfl_xor(s, XR);
+    if (!in || m >= p.M) return;
+    const int G = p.K / 64, g = hg >> 1, h = hg & 1;
+    q35_xw_store(reinterpret_cast<uint8_t *>(p.xw) + q35_xw_block(m, g, G), 32 * h + (m & 31), v[0], v[1], s, mx);
+    if (h == 0) p.xsum[(size_t)g * p.Mpad + m] = s2;
 }
 
-/* (16 s, b - 16 s) of a weight's rows and groups as [G][npad] (zeros for
- * rows past N), from its BF16 scales and biases [N][G] (biases may be
- * NULL) */
+/* A weight's s (fp32) and b (BF16, zeros for NULL biases) as two [G][npad]
+ * tables, zeros for rows past N, from its BF16 scales and biases [N][G] */
 __global__ void sb_kernel(const uint16_t *scales, const uint16_t *biases, Q35Mlx4SB *sb, int N, int G,
                           int npad) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)G * npad) return;
+    const int64_t n_all = (int64_t)G * npad, i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_all) return;
     const int g = (int)(i / npad), n = (int)(i % npad);
-    float sv = 0.0f, bv = 0.0f;
-    if (n < N) {
-        const float s = q35_bf2f(scales[(size_t)n * G + g]);
-        const float b = biases ? q35_bf2f(biases[(size_t)n * G + g]) : 0.0f;
-        sv = QSTEP * s;
-        bv = b - sv;
-    }
-    sb[i] = Q35Mlx4SB{sv, bv};
+    float *s = reinterpret_cast<float *>(sb);
+    uint16_t *b = reinterpret_cast<uint16_t *>(s + n_all);
+    s[i] = n < N ? q35_bf2f(scales[(size_t)n * G + g]) : 0.0f;
+    b[i] = n < N && biases ? biases[(size_t)n * G + g] : (uint16_t)0;
+}
+
+/* Where a lane's 32 nibbles (fields f = 0..31, q35_xw_col) lie in its 16
+ * bytes.  16 fp6 fields are 96 bits whose values occupy M0 of the first dword, M1
+ * of the second and (~M0 | ~M1) of the third: 22 + 22 + 20 bits.  Two
+ * packed dwords A and B hold the first two in place and, in the bits those
+ * leave, the third's, so that the operand is A & M0, B & M1 and
+ * (A & ~M0) | (B & ~M1). */
+constexpr uint32_t M0 = 0xcf3cf3cfu, M1 = 0xf3cf3cf3u;
+__device__ __forceinline__ i32x8_t expand_fp6(u32x4_t w) {
+    return i32x8_t{(int)(w[0] & M0), (int)(w[1] & M1), (int)((w[0] & ~M0) | (w[1] & ~M1)),
+                   (int)(w[2] & M0), (int)(w[3] & M1), (int)((w[2] & ~M0) | (w[3] & ~M1)), 0, 0};
 }
 
 /* the weight words [N][K/8] as wt blocks [npad/256][G][512 granules of
- * 16 bytes]: granule p of block (tile, g) = words 4 wslot(r, p % 2) ..
- * +3 of group g of row tile * 256 + r, r = p / 2; zeros past N */
+ * 16 bytes]: granule p of block (tile, g) is half wslot(r, p % 2) of group g of
+ * row tile * 256 + r, r = p / 2, packed as above; zeros past N */
 __global__ void wt_kernel(const uint32_t *vals, u32x4_t *wt, int N, int K, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -206,34 +182,65 @@ __global__ void wt_kernel(const uint32_t *vals, u32x4_t *wt, int N, int K, int64
     const int64_t blk = i >> 9;
     const int g = (int)(blk % G), tile = (int)(blk / G);
     const int r = p >> 1, row = tile * NTILE + r;
-    u32x4_t v = {0u, 0u, 0u, 0u};
-    if (row < N)
-        v = *reinterpret_cast<const u32x4_t *>(vals + (size_t)row * (K / 8) + 8 * g + 4 * wslot(r, p & 1));
-    wt[i] = v;
+    u32x4_t o = {0u, 0u, 0u, 0u};
+    if (row < N) {
+        const u32x4_t v =
+            *reinterpret_cast<const u32x4_t *>(vals + (size_t)row * (K / 8) + 8 * g + 4 * wslot(r, p & 1));
+#pragma unroll
+        for (int f = 0; f < 32; f++) {
+            const int k = q35_xw_col(f);
+            const uint32_t q = (v[k >> 3] >> (4 * (k & 7))) & 15u;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int pos = 6 * (f & 15) + j, b = pos & 31;
+                const int src = pos < 32 ? 0 : pos < 64 ? 1 : (int)((M0 >> b) & 1);
+                o[2 * (f >> 4) + src] |= ((q >> j) & 1u) << b;
+            }
+        }
+    }
+    wt[i] = o;
 }
 
-/* a word's 8 nibbles as the fp16 B operand 1 + q / 16, in word order:
- * pair j (nibbles j and j + 4, bits 4j and 16 + 4j) shifted to bits 6 and
- * 22, masked, ORed into the exponent of 1.  The mask and the exponent bits
- * are held in registers (an SGPR and a VGPR) so that each pair is one
- * shift and one v_and_or_b32. */
-__device__ __forceinline__ f16x8_t nib_f16(uint32_t w, uint32_t mask, uint32_t one) {
-    u32x4_t u;
-    u[0] = ((w << 6) & mask) | one;
-    u[1] = ((w << 2) & mask) | one;
-    u[2] = ((w >> 2) & mask) | one;
-    u[3] = ((w >> 6) & mask) | one;
-    return __builtin_bit_cast(f16x8_t, u);
+/* an operand's 24 bytes from the 16 + 8 they are stored as; the builtin takes
+ * eight dwords and reads six */
+__device__ __forceinline__ i32x8_t fp6_operand(u32x4_t x4, u32x2_t x2) {
+    return i32x8_t{(int)x4[0], (int)x4[1], (int)x4[2], (int)x4[3], (int)x2[0], (int)x2[1], 0, 0};
 }
-
-__device__ __forceinline__ int ntiles(int N) { return (N + NTILE - 1) / NTILE; }
+/* part + digit d x nibbles over a group.  Digit d's exponent is byte d % 4 of
+ * ex[d / 4]; the nibble codes' unit is 1/8. */
+template <int d>
+__device__ __forceinline__ f32x16_t mfma_digit(i32x8_t x, u32x2_t ex, i32x8_t w, f32x16_t part) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, w, part, 2, 2, d & 3, (int)ex[d >> 2], 0, 130);
+}
+/* a lane's X of one group, and the group's product with a weight operand, the
+ * lowest digit first */
+struct XDigits {
+    i32x8_t d[Q35_XW_DIGITS];
+    u32x2_t ex;
+};
+__device__ __forceinline__ f32x16_t group_product(const XDigits &x, i32x8_t w) {
+    f32x16_t t;
+#pragma unroll
+    for (int i = 0; i < 16; i++) t[i] = 0.0f;
+    t = mfma_digit<4>(x.d[4], x.ex, w, t);
+    t = mfma_digit<3>(x.d[3], x.ex, w, t);
+    t = mfma_digit<2>(x.d[2], x.ex, w, t);
+    t = mfma_digit<1>(x.d[1], x.ex, w, t);
+    return mfma_digit<0>(x.d[0], x.ex, w, t);
+}
 
 /* One workgroup per (job, 256-feature tile, 64-token tile), numbered with
  * the token tile fastest over the jobs' feature tiles in order.  Work-
  * groups are handed to the 8 XCDs in turn, so with 8 | token tiles an XCD
- * holds token tiles of one residue mod 8 over consecutive feature tiles:
- * about 8 x 8 tiles at once, sharing X and weight tiles in its L2. */
-__global__ __launch_bounds__(NT, 2) void gemm_kernel(Q35Mlx4Gemm p) {
+ * holds token tiles of one residue mod 8 over consecutive feature tiles,
+ * sharing X and weight tiles in its L2. */
+template <int V>
+struct Int {
+    static constexpr int value = V;
+};
+constexpr int NW = 4;                  /* waves, 2 along the tokens x 2 along the features */
+constexpr int OFF_W = 2 * XBLK, OFF_S = OFF_W + WBLK, STAGE = OFF_S + NTILE * 4, NSTAGE = 3;
+__global__ __launch_bounds__(64 * NW, 2) void gemm_kernel(Q35Mlx4Gemm p) {
     const int ntm = p.Mpad / MT;
     const int mt = blockIdx.x % ntm;
     int nt = blockIdx.x / ntm;
@@ -242,17 +249,16 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(Q35Mlx4Gemm p) {
     Q35Mlx4GemmJob J = p.jobs[0];
 #pragma unroll
     for (int j = 1; j < Q35_GEMM_MAX_JOBS; j++) {
-        const int prev = ntiles(J.N);
+        const int prev = (J.N + NTILE - 1) / NTILE;
         if (j < p.njobs && nt >= prev) {
             nt -= prev;
             J = p.jobs[j];
         }
     }
-    float *const Y = J.y;
-    const int ldy = J.ldy;
     const int n0 = nt * NTILE, m0 = mt * MT;
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int mb = w & 1, nw = w >> 1;
     const int h = lane >> 5, c = lane & 31;
     const int G = p.K / 64;
     const int npad = (J.N + NTILE - 1) / NTILE * NTILE;
@@ -265,169 +271,250 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(Q35Mlx4Gemm p) {
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<uint32_t *>(J.vals)), 0, (int)((size_t)npad * p.K / 2), Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
-        q35_uniform_ptr(const_cast<Q35Mlx4SB *>(J.sb)), 0, (int)((size_t)G * npad * 8), Q35_BUF_DW3);
+        q35_uniform_ptr(const_cast<Q35Mlx4SB *>(J.sb)), 0, (int)((size_t)G * npad * 4), Q35_BUF_DW3);
+    const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr((char *)const_cast<Q35Mlx4SB *>(J.sb) + (size_t)G * npad * 4), 0,
+        (int)((size_t)G * npad * 2), Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t ssr = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<float *>(p.xsum)), 0, (int)((size_t)G * p.Mpad * 4), Q35_BUF_DW3);
 
-    /* group g into stage st: X 16 loads, weights 8, (s, b') 2, xsum 1 (a
-     * dword load); waves 0-2 issue 7 of them, wave 3 issues 6 */
-    auto issue = [&](int g, int st) {
-        const uint32_t sb = lds0 + (uint32_t)(st * STAGE);
-        const uint32_t xb = (uint32_t)(mt * G + g) * (2 * XBLK);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int i = w + 4 * q;
-            q35_dma16(xr, sb + i * 1024, lane * 16, xb + i * 1024);
+    /* load q of group g into stage st: X (a wave 16 / NW copies of 1 KB), the
+     * weight (2 copies), s (256 bytes).  Groups past the last are addressed
+     * out of range: no memory access, and the count of loads stays. */
+    constexpr int XL = 16 / NW, LOADS = XL + 3;
+    auto issue = [&](int q, int g, int st) {
+        const uint32_t sb = lds0 + (uint32_t)(st * STAGE), past = g < G ? 0u : 0x80000000u;
+        if (q < XL) {
+            const int i = w + NW * q;
+            q35_dma16(xr, sb + i * 1024, lane * 16 + past,
+                      (uint32_t)((2 * mt + (i >> 3)) * G + g) * XBLK + (i & 7) * 1024);
+        } else if (q < XL + 2) {
+            const int i = w + NW * (q - XL);
+            q35_dma16(wr, sb + OFF_W + i * 1024, lane * 16 + past,
+                      (uint32_t)(nt * G + g) * WBLK + i * 1024);
+        } else {
+            q35_dma4(sr, sb + OFF_S + w * 256, lane * 4 + past, (uint32_t)(g * npad + n0) * 4 + w * 256);
         }
-        const uint32_t wb = (uint32_t)(nt * G + g) * WBLK;
+    };
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int i = w + 4 * q;
-            q35_dma16(wr, sb + OFF_W + i * 1024, lane * 16, wb + i * 1024);
+    for (int g = 0; g < 3; g++)
+#pragma unroll
+        for (int q = 0; q < LOADS; q++) issue(q, g, g);
+
+    f32x16_t acc[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[nb][i] = 0.0f;
+    /* a wave whose features all lie past N (a narrow job) only stages */
+    const bool idle = n0 + 128 * nw >= J.N;
+    /* sum_g b xsum, 16 groups a step (lane half h: groups 8h ..; groups past
+     * G read as zeros on both sides) */
+    if (!idle) {
+        for (int g0 = 0; g0 < G; g0 += 16) {
+            float xs[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                xs[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    ssr, ((8 * h + j) * p.Mpad + m0 + 32 * mb + c) * 4, g0 * p.Mpad * 4, 0));
+            bf16x8_t b[4];
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    b[nb][j] = q35_as_bf16(__builtin_amdgcn_raw_buffer_load_b16(
+                        br, ((8 * h + j) * npad + n0 + 128 * nw + 32 * nb + c) * 2, g0 * npad * 2, 0));
+            bf16x8_t x0, x1, x2;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                x0[j] = (__bf16)xs[j];
+                const float r1 = xs[j] - (float)x0[j];
+                x1[j] = (__bf16)r1;
+                x2[j] = (__bf16)(r1 - (float)x1[j]);
+            }
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++) {
+                acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x2, b[nb], acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x1, b[nb], acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x0, b[nb], acc[nb], 0, 0, 0);
+            }
         }
-        if (w < 2)
-            q35_dma16(sr, sb + OFF_SB + w * 1024, lane * 16, (uint32_t)(g * npad + n0) * 8 + w * 1024);
-        else if (w == 2)
-            q35_dma4(ssr, sb + OFF_XS, lane * 4, (uint32_t)(g * p.Mpad + m0) * 4);
-    };
-    /* this wave's loads of the group before the last issued have landed */
-    auto wait_prev = [&]() {
-        if (w == 3)
-            q35_wait_vm<6>();
-        else
-            q35_wait_vm<7>();
-    };
-
-    f32x16_t acc[2][2];
-#pragma unroll
-    for (int mb = 0; mb < 2; mb++)
-#pragma unroll
-        for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[mb][nb][i] = 0.0f;
-
-    issue(0, 0);
-    if (G > 1) {
-        issue(1, 1);
-        wait_prev();
-    } else {
-        q35_wait_vm<0>();
     }
+
+    /* The wave's four blocks in two pairs, a pair's MFMAs digit by digit (two
+     * independent chains).  Between a pair's MFMAs go the fp32 scaling of the
+     * pair before it, the LDS reads and the expansion of the next pair's
+     * weight, and under the second pair the next group's X, digit by digit as
+     * this group's is last used.  So the stage of group g is last read in the
+     * first pair of group g: the barrier between the pairs frees it for group
+     * g + 3, and publishes group g + 1.  Left to itself the scheduler puts a
+     * block's scaling and expansion behind its own five MFMAs, so the order is
+     * pinned step by step. */
+    const uint32_t xo = (uint32_t)(mb * XBLK + lane * 16), xo2 = (uint32_t)(mb * XBLK + lane * 8);
+    auto lds_x = [&](int st, int d) {
+        const uint8_t *S = smem + st * STAGE + d * Q35_XW_DIG;
+        return fp6_operand(*reinterpret_cast<const u32x4_t *>(S + xo),
+                           *reinterpret_cast<const u32x2_t *>(S + xo2 + 1024));
+    };
+    auto lds_ex = [&](int st) {
+        return *reinterpret_cast<const u32x2_t *>(smem + st * STAGE + xo2 + Q35_XW_EXP);
+    };
+    const int r0 = 128 * nw + c;
+    const uint32_t wo = OFF_W + r0 * 32 + wslot(r0, h) * 16;   /* wslot is the same 32 rows on */
+    auto lds_w = [&](int st, int nb) {
+        return *reinterpret_cast<const u32x4_t *>(smem + st * STAGE + wo + nb * 1024);
+    };
+    auto lds_s = [&](int st, int nb) {
+        return *reinterpret_cast<const float *>(smem + st * STAGE + OFF_S + (r0 + 32 * nb) * 4);
+    };
+    auto scale = [&](int nb, float sc, const f32x16_t &part, auto lo, auto hi) {
+#pragma unroll
+        for (int i = decltype(lo)::value; i < decltype(hi)::value; i++) acc[nb][i] = fmaf(sc, part[i], acc[nb][i]);
+    };
+    using I0 = Int<0>;
+    using I6 = Int<6>;
+    using I11 = Int<11>;
+    using I16 = Int<16>;
+    /* the values up to here computed before anything after: an empty volatile
+     * asm claims to change them (register operations are otherwise free to
+     * move across sched_barrier when the blocks are selected) */
+    auto hold = [](f32x16_t &a, f32x16_t &b) { asm volatile("" : "+v"(a), "+v"(b)); };
+    auto pin = [] { __builtin_amdgcn_sched_barrier(0); };
+    f32x16_t zero;
+#pragma unroll
+    for (int i = 0; i < 16; i++) zero[i] = 0.0f;
+
+    q35_wait_vm<2 * LOADS>();
     q35_lds_barrier();
-
-    /* a wave whose 64 features all lie past N (a narrow job) only stages */
-    const bool idle = n0 + 64 * w >= J.N;
-    uint32_t mask, one;
-    asm("s_mov_b32 %0, 0x03c003c0" : "=s"(mask));
-    asm("v_mov_b32 %0, 0x3c003c00" : "=v"(one));
-
+    if (idle) {
+        for (int g = 0; g < G; g++) {
+            q35_wait_vm<LOADS>();
+            q35_lds_barrier();
+#pragma unroll
+            for (int q = 0; q < LOADS; q++) issue(q, g + 3, g % 3);
+        }
+        q35_wait_vm<0>();
+        return;
+    }
+    i32x8_t x[Q35_XW_DIGITS];
+#pragma unroll
+    for (int d = 0; d < Q35_XW_DIGITS; d++) x[d] = lds_x(0, d);
+    u32x2_t ex = lds_ex(0);
+    i32x8_t w0 = expand_fp6(lds_w(0, 0)), w1 = expand_fp6(lds_w(0, 1));
+    float sa0 = lds_s(0, 0), sa1 = lds_s(0, 1), sb0 = 0.0f, sb1 = 0.0f;
+    f32x16_t pa0, pa1, pb0 = zero, pb1 = zero;
     int st = 0;
     for (int g = 0; g < G; g++) {
-        if (g + 2 < G) issue(g + 2, st == 0 ? 2 : st - 1);
-        if (!idle) {
-            const uint8_t *S = smem + st * STAGE;
-            /* the weight operand: this lane's words 4h..4h+3 of rows
-             * 64w + 32nb + c, and their (s, b') */
-            f16x8_t bf[2][4];
-            float sc[2], bp[2];
-#pragma unroll
-            for (int nb = 0; nb < 2; nb++) {
-                const int r = 64 * w + 32 * nb + c;
-                const u32x4_t wq = *reinterpret_cast<const u32x4_t *>(S + OFF_W + r * 32 + wslot(r, h) * 16);
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) bf[nb][ks] = nib_f16(wq[ks], mask, one);
-                const float2 v = *reinterpret_cast<const float2 *>(S + OFF_SB + r * 8);
-                sc[nb] = v.x;
-                bp[nb] = v.y;
-            }
-
-            /* acc += b' * xsum first: it does not wait for the MFMAs, so it
-             * runs while the previous wave's MFMAs hold the pipe */
-            {
-                const float *xs0 = reinterpret_cast<const float *>(S + OFF_XS);
-#pragma unroll
-                for (int mb = 0; mb < 2; mb++) {
-                    float xsv[16];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const float4 v = *reinterpret_cast<const float4 *>(xs0 + 32 * mb + 8 * q + 4 * h);
-                        xsv[4 * q] = v.x, xsv[4 * q + 1] = v.y, xsv[4 * q + 2] = v.z, xsv[4 * q + 3] = v.w;
-                    }
-#pragma unroll
-                    for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-                        for (int i = 0; i < 16; i++) acc[mb][nb][i] = fmaf(bp[nb], xsv[i], acc[mb][nb][i]);
-                }
-            }
-            /* the group's MFMAs at raised wave priority, so that the SIMD's
-             * other wave does its VALU work around them rather than
-             * competing for the issue slot (output GEMM 126 -> 116 us) */
-            __builtin_amdgcn_s_setprio(1);
-            f32x16_t tmp[2][2];
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                f16x8_t ah[2], al[2];
-#pragma unroll
-                for (int mb = 0; mb < 2; mb++) {
-                    const int off = ((mb * 4 + ks) * 64 + lane) * 16;
-                    ah[mb] = *reinterpret_cast<const f16x8_t *>(S + off);
-                    al[mb] = *reinterpret_cast<const f16x8_t *>(S + XBLK + off);
-                }
-#pragma unroll
-                for (int mb = 0; mb < 2; mb++)
-#pragma unroll
-                    for (int nb = 0; nb < 2; nb++) {
-                        if (ks == 0) {
-                            f32x16_t z;
-#pragma unroll
-                            for (int i = 0; i < 16; i++) z[i] = 0.0f;
-                            tmp[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[mb], bf[nb][ks], z, 0, 0, 0);
-                        } else {
-                            tmp[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[mb], bf[nb][ks],
-                                                                                 tmp[mb][nb], 0, 0, 0);
-                        }
-                        tmp[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[mb], bf[nb][ks], tmp[mb][nb], 0, 0, 0);
-                    }
-            }
-            __builtin_amdgcn_s_setprio(0);
-            /* acc += s' * partial; lane rows 32mb + 8(i/4) + 4h + i%4 */
-#pragma unroll
-            for (int mb = 0; mb < 2; mb++)
-#pragma unroll
-                for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[mb][nb][i] = fmaf(sc[nb], tmp[mb][nb][i], acc[mb][nb][i]);
-        }
-        /* the next group's stage is complete for every wave; this one is
-         * free for the load issued next iteration */
-        if (g + 2 < G)
-            wait_prev();
-        else
-            q35_wait_vm<0>();
+        const int sn = st == 2 ? 0 : st + 1;
+        /* blocks 0 and 1; the scaling of blocks 2 and 3 of the group before */
+        pa0 = mfma_digit<4>(x[4], ex, w0, zero);
+        pa1 = mfma_digit<4>(x[4], ex, w1, zero);
+        u32x4_t q0 = lds_w(st, 2), q1 = lds_w(st, 3);
+        float t0 = lds_s(st, 2), t1 = lds_s(st, 3);
+        hold(pa0, pa1);
+        pin();
+        pa0 = mfma_digit<3>(x[3], ex, w0, pa0);
+        pa1 = mfma_digit<3>(x[3], ex, w1, pa1);
+        scale(2, sb0, pb0, I0{}, I11{});
+        hold(pa0, pa1);
+        hold(acc[2], acc[3]);
+        pin();
+        pa0 = mfma_digit<2>(x[2], ex, w0, pa0);
+        pa1 = mfma_digit<2>(x[2], ex, w1, pa1);
+        scale(2, sb0, pb0, I11{}, I16{});
+        scale(3, sb1, pb1, I0{}, I6{});
+        hold(pa0, pa1);
+        hold(acc[2], acc[3]);
+        pin();
+        pa0 = mfma_digit<1>(x[1], ex, w0, pa0);
+        pa1 = mfma_digit<1>(x[1], ex, w1, pa1);
+        scale(3, sb1, pb1, I6{}, I16{});
+        hold(pa0, pa1);
+        hold(acc[2], acc[3]);
+        pin();
+        pa0 = mfma_digit<0>(x[0], ex, w0, pa0);
+        pa1 = mfma_digit<0>(x[0], ex, w1, pa1);
+        w0 = expand_fp6(q0);
+        w1 = expand_fp6(q1);
+        sb0 = t0;
+        sb1 = t1;
+        hold(pa0, pa1);
+        pin();
+        q35_wait_vm<LOADS>();                     /* group g + 1 */
         q35_lds_barrier();
-        st = st == 2 ? 0 : st + 1;
+        pin();
+        /* blocks 2 and 3; the scaling of blocks 0 and 1; X of group g + 1 */
+        pb0 = mfma_digit<4>(x[4], ex, w0, zero);
+        pb1 = mfma_digit<4>(x[4], ex, w1, zero);
+        x[4] = lds_x(sn, 4);
+        const u32x2_t exn = lds_ex(sn);
+        q0 = lds_w(sn, 0);
+        q1 = lds_w(sn, 1);
+        t0 = lds_s(sn, 0);
+        t1 = lds_s(sn, 1);
+        hold(pb0, pb1);
+        pin();
+#pragma unroll
+        for (int q = 0; q < 2; q++) issue(q, g + 3, st);
+        pb0 = mfma_digit<3>(x[3], ex, w0, pb0);
+        pb1 = mfma_digit<3>(x[3], ex, w1, pb1);
+        x[3] = lds_x(sn, 3);
+        scale(0, sa0, pa0, I0{}, I11{});
+        hold(pb0, pb1);
+        hold(acc[0], acc[1]);
+        pin();
+#pragma unroll
+        for (int q = 2; q < 4; q++) issue(q, g + 3, st);
+        pb0 = mfma_digit<2>(x[2], ex, w0, pb0);
+        pb1 = mfma_digit<2>(x[2], ex, w1, pb1);
+        x[2] = lds_x(sn, 2);
+        scale(0, sa0, pa0, I11{}, I16{});
+        scale(1, sa1, pa1, I0{}, I6{});
+        hold(pb0, pb1);
+        hold(acc[0], acc[1]);
+        pin();
+#pragma unroll
+        for (int q = 4; q < LOADS; q++) issue(q, g + 3, st);
+        pb0 = mfma_digit<1>(x[1], ex, w0, pb0);
+        pb1 = mfma_digit<1>(x[1], ex, w1, pb1);
+        x[1] = lds_x(sn, 1);
+        scale(1, sa1, pa1, I6{}, I16{});
+        hold(pb0, pb1);
+        hold(acc[0], acc[1]);
+        pin();
+        pb0 = mfma_digit<0>(x[0], ex, w0, pb0);
+        pb1 = mfma_digit<0>(x[0], ex, w1, pb1);
+        x[0] = lds_x(sn, 0);
+        w0 = expand_fp6(q0);
+        w1 = expand_fp6(q1);
+        sa0 = t0;
+        sa1 = t1;
+        ex = exn;
+        hold(pb0, pb1);
+        pin();
+        st = sn;
     }
+    scale(2, sb0, pb0, I0{}, I16{});
+    scale(3, sb1, pb1, I0{}, I16{});
+    q35_wait_vm<0>();
 
-    int nrow[2];
-#pragma unroll
-    for (int nb = 0; nb < 2; nb++) nrow[nb] = n0 + 64 * w + 32 * nb + c;
     /* y[m][n] (+= with accumulate): lanes 0..31 of a row write 32
-     * consecutive features */
+     * consecutive features; lane rows 8(i/4) + 4h + i%4 */
+    float *const Y = J.y;
+    const int ldy = J.ldy;
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++)
+    for (int nb = 0; nb < 4; nb++) {
+        const int n = n0 + 128 * nw + 32 * nb + c;
+        if (n >= J.N) continue;
 #pragma unroll
-        for (int nb = 0; nb < 2; nb++) {
-            const int n = nrow[nb];
-            if (n >= J.N) continue;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int m = m0 + 32 * mb + 8 * (i >> 2) + 4 * h + (i & 3);
-                if (m < p.M) {
-                    float *dst = Y + (size_t)m * ldy + n;
-                    *dst = p.accumulate ? *dst + acc[mb][nb][i] : acc[mb][nb][i];
-                }
+        for (int i = 0; i < 16; i++) {
+            const int m = m0 + 32 * mb + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (m < p.M) {
+                float *dst = Y + (size_t)m * ldy + n;
+                *dst = p.accumulate ? *dst + acc[nb][i] : acc[nb][i];
             }
         }
+    }
 }
 
 /* ---- the same product for chunks of few tokens ----------------------------
@@ -441,14 +528,16 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(Q35Mlx4Gemm p) {
  * order, the weight words in the stage order, both whole lines), with no
  * LDS staging and no barrier in the loop.  The waves' partial tiles meet in
  * LDS and are added in wave order, so a result does not depend on timing.
- * The bias term b' xsum is an fp32 MFMA over the wave's group pairs
+ * The bias term b xsum is an fp32 MFMA over the wave's group pairs
  * (v_mfma_f32_32x32x2_f32: one group a lane half) on its own accumulator.
  * What bounds it: a CU's 64 B a cycle from L2, (MB K 128 + NB K 20) bytes a
  * workgroup.  Feature tiles are dealt to the XCDs (id mod 8) with the token
  * tiles of one feature tile behind each other, so an XCD's L2 fetches a
  * weight tile once. */
-template <int MB, int NB, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_few_kernel(Q35Mlx4Gemm p, int nft) {
+constexpr int FEW_WAVES = 8;
+template <int MB, int NB>
+__global__ __launch_bounds__(64 * FEW_WAVES) void gemm_few_kernel(Q35Mlx4Gemm p, int nft) {
+    constexpr int NW = FEW_WAVES;
     const int ntm = (p.M + 32 * MB - 1) / (32 * MB);
     const int q = blockIdx.x >> 3, mt = q % ntm;
     int nt = (q / ntm) * 8 + (blockIdx.x & 7);
@@ -476,16 +565,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(Q35Mlx4Gemm p, int nf
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<uint32_t *>(J.vals)), 0, (int)((size_t)npad * p.K / 2), Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
-        q35_uniform_ptr(const_cast<Q35Mlx4SB *>(J.sb)), 0, (int)((size_t)G * npad * 8), Q35_BUF_DW3);
+        q35_uniform_ptr(const_cast<Q35Mlx4SB *>(J.sb)), 0, (int)((size_t)G * npad * 4), Q35_BUF_DW3);
+    const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr((char *)const_cast<Q35Mlx4SB *>(J.sb) + (size_t)G * npad * 4), 0,
+        (int)((size_t)G * npad * 2), Q35_BUF_DW3);
     const __amdgpu_buffer_rsrc_t ssr = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<float *>(p.xsum)), 0, (int)((size_t)G * p.Mpad * 4), Q35_BUF_DW3);
-    uint32_t mask, one;
-    asm("s_mov_b32 %0, 0x03c003c0" : "=s"(mask));
-    asm("v_mov_b32 %0, 0x3c003c00" : "=v"(one));
-
-    /* one group's operands: X hi and lo, weight words, s' */
+    /* one group's operands: X, the weight's nibbles, s */
     struct Ops {
-        u32x4_t xh[MB][4], xl[MB][4], wq[NB];
+        XDigits x[MB];
+        u32x4_t wq[NB];
         float sc[NB];
     };
     int wrow[NB];
@@ -494,21 +583,24 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(Q35Mlx4Gemm p, int nf
         const int rr = (n0 & (NTILE - 1)) + 32 * nb + c;
         wrow[nb] = (rr * 2 + wslot(rr, h)) * 16;
     }
-    const int mt64 = m0 / MT, mb0 = (m0 / 32) & 1, tile = n0 / NTILE;
+    const int tile = n0 / NTILE;
     auto load = [&](int g, Ops &o) {
-        const int xb = (mt64 * G + g) * (2 * XBLK) + mb0 * (XBLK / 2);
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
+        for (int mb = 0; mb < MB; mb++) {
+            const int xb = ((m0 / 32 + mb) * G + g) * XBLK;
+            o.x[mb].ex = __builtin_amdgcn_raw_buffer_load_b64(xr, lane * 8 + Q35_XW_EXP, xb, 0);
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                o.xh[mb][ks] = __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16 + ks * 1024, xb + mb * 4096, 0);
-                o.xl[mb][ks] = __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16 + ks * 1024, xb + XBLK + mb * 4096, 0);
+            for (int d = Q35_XW_DIGITS - 1; d >= 0; d--) {
+                o.x[mb].d[d] = fp6_operand(
+                    __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16 + d * Q35_XW_DIG, xb, 0),
+                    __builtin_amdgcn_raw_buffer_load_b64(xr, lane * 8 + d * Q35_XW_DIG + 1024, xb, 0));
             }
+        }
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
             o.wq[nb] = __builtin_amdgcn_raw_buffer_load_b128(wr, wrow[nb], (tile * G + g) * WBLK, 0);
             o.sc[nb] = __uint_as_float(
-                __builtin_amdgcn_raw_buffer_load_b32(sr, (32 * nb + c) * 8, (g * npad + n0) * 8, 0));
+                __builtin_amdgcn_raw_buffer_load_b32(sr, (32 * nb + c) * 4, (g * npad + n0) * 4, 0));
         }
     };
 
@@ -521,28 +613,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(Q35Mlx4Gemm p, int nf
             for (int i = 0; i < 16; i++) acc[mb][nb][i] = 0.0f;
 
     auto multiply = [&](const Ops &o) {
-        f16x8_t bf[NB][4];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++)
+        for (int nb = 0; nb < NB; nb++) {
+            const i32x8_t wf = expand_fp6(o.wq[nb]);
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) bf[nb][ks] = nib_f16(o.wq[nb][ks], mask, one);
+            for (int mb = 0; mb < MB; mb++) {
+                const f32x16_t part = group_product(o.x[mb], wf);
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                f32x16_t tmp;
-#pragma unroll
-                for (int i = 0; i < 16; i++) tmp[i] = 0.0f;
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    tmp = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, o.xh[mb][ks]),
-                                                                 bf[nb][ks], tmp, 0, 0, 0);
-                    tmp = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, o.xl[mb][ks]),
-                                                                 bf[nb][ks], tmp, 0, 0, 0);
-                }
-#pragma unroll
-                for (int i = 0; i < 16; i++) acc[mb][nb][i] = fmaf(o.sc[nb], tmp[i], acc[mb][nb][i]);
+                for (int i = 0; i < 16; i++) acc[mb][nb][i] = fmaf(o.sc[nb], part[i], acc[mb][nb][i]);
             }
+        }
     };
     /* this wave's group pairs; an odd G's missing group reads zeros */
     for (int g = 2 * w; g < G; g += 2 * NW) {
@@ -554,8 +634,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_few_kernel(Q35Mlx4Gemm p, int nf
                 ssr, gh < G ? (gh * p.Mpad + m0 + 32 * mb + c) * 4 : (int)0x80000000, 0, 0));
 #pragma unroll
         for (int nb = 0; nb < NB; nb++)
-            bs[nb] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                sr, gh < G ? (gh * npad + n0 + 32 * nb + c) * 8 + 4 : (int)0x80000000, 0, 0));
+            bs[nb] = q35_bf2f(__builtin_amdgcn_raw_buffer_load_b16(
+                br, gh < G ? (gh * npad + n0 + 32 * nb + c) * 2 : (int)0x80000000, 0, 0));
         Ops a, b;
         const bool two = g + 1 < G;
         load(g, a);
@@ -611,38 +691,41 @@ inline int64_t few_tiles(const Q35Mlx4Gemm *p, int MB, int NB) {
     return n * ((p->M + 32 * MB - 1) / (32 * MB));
 }
 
-/* Which kernel a product runs on: 0 gemm_kernel, 1..4 gemm_few_kernel at
- * 32 x 32, 32 x 64 and 64 x 64 with 8 waves, 64 x 64 with 4.  The smallest
- * tile whose workgroups are at most one a CU (smaller tiles read X more
- * often, a second round costs as much as the first); past that two 4-wave
- * workgroups share a CU; and from 140 64 x 64 x 64 products a CU on,
- * gemm_kernel, whose workgroups share X through LDS, is faster.  us a launch
- * (projections 12352 x 2048 | output 2048 x 4096), gemm_kernel -> here:
- *   M =   32: 40.9 ->  8.3 | 75.6 ->  8.8     M =  256: 42.8 -> 36.9 | 77.2 -> 13.1
- *   M =   64: 41.3 -> 12.1 | 76.3 ->  8.9     M =  512: 55.0 (66.9)  | 76.0 -> 22.3
- *   M =  128: 42.0 -> 20.4 | 76.8 ->  9.8     M = 1024: 107.7 (139)  | 78.2 -> 45.8
- * (in brackets the form that is not taken). */
+/* Which kernel a product runs on: 0 gemm_kernel, 1..3 gemm_few_kernel at
+ * 32 x 32, 32 x 64 and 64 x 64.  The smallest tile whose workgroups are at
+ * most one a CU (smaller tiles read X more often, a second round costs as
+ * much as the first).  From 600 64 x 64 tiles on (2.3 a CU), gemm_kernel, whose
+ * workgroups share X through LDS, is faster at both widths.  us a launch,
+ * gemm_few_kernel (the form taken) | gemm_kernel:
+ *   projections 12352 x 2048       output 2048 x 4096
+ *   M =   32:  7.9 | 27.7            9.3 | 47.2
+ *   M =   64: 12.0 | 27.6            9.8 | 47.8
+ *   M =  128: 21.0 | 28.2           10.2 | 48.3
+ *   M =  192: 29.4 | 29.4           11.1 | 48.3
+ *   M =  256: 37.5 | 30.8           12.1 | 48.5
+ *   M =  512: 69.2 | 45.9           21.2 | 49.1
+ *   M = 1024:  148 | 82.1           46.2 | 50.6
+ *   M = 1536:  306 | 117            90.7 | 52.8 */
 inline int few_tokens(const Q35Mlx4Gemm *p) {
     constexpr int64_t CUS = 256;
     for (int j = 0; j < p->njobs; j++)
         if (p->jobs[j].N % 4 != 0) return 0;    /* its stores are four features wide */
-    const int64_t t22 = few_tiles(p, 2, 2);
-    if (t22 * (p->K / 64) > 140 * CUS) return 0;
+    if (few_tiles(p, 2, 2) > 600) return 0;
     if (few_tiles(p, 1, 1) <= CUS) return 1;
     if (few_tiles(p, 1, 2) <= CUS) return 2;
     /* half of the last 64-row tile would be padding, at least a fifth of
-     * the work (M = 96, GQA projections: 14.4 us against 19.5) */
+     * the work (M = 96, GQA projections: 13.3 us against 20.2) */
     if (p->M > 64 && p->M <= 160 && p->M % 64 > 0 && p->M % 64 <= 32) return 2;
-    return t22 <= CUS ? 3 : 4;
+    return 3;
 }
 
-template <int MB, int NB, int NW>
+template <int MB, int NB>
 hipError_t launch_few(const Q35Mlx4Gemm *p, hipStream_t stream) {
     int64_t nft = 0;
     for (int j = 0; j < p->njobs; j++) nft += (p->jobs[j].N + 32 * NB - 1) / (32 * NB);
     const int64_t grid = (nft + 7) / 8 * 8 * ((p->M + 32 * MB - 1) / (32 * MB));
     if (grid >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_few_kernel<MB, NB, NW>), dim3((unsigned)grid), dim3(64 * NW), 0, stream, *p, (int)nft);
+    hipLaunchKernelGGL((gemm_few_kernel<MB, NB>), dim3((unsigned)grid), dim3(64 * FEW_WAVES), 0, stream, *p, (int)nft);
     return hipGetLastError();
 }
 
@@ -668,18 +751,16 @@ extern "C" hipError_t q35_mlx4_wt(const uint32_t *vals, uint32_t *wt, int N, int
 }
 
 namespace {
-/* XR rows a workgroup of N1 threads for K <= 2048 (256 words a row), N2 for
- * K <= 4096, 1024 for K <= 8192, as many words a thread as that takes */
-template <int XR, int N1, int N2>
+/* XR rows a workgroup, 32 columns a thread */
+template <int XR>
 void launch_xprep(const Q35Mlx4Xprep *p, hipStream_t stream) {
-    const int words = p->K / 8;
     const dim3 grid((p->M + XR - 1) / XR);
-    if (words <= 256)
-        hipLaunchKernelGGL((xprep_kernel<N1, XR, 256 * XR / N1>), grid, dim3(N1), 0, stream, *p);
-    else if (words <= 512)
-        hipLaunchKernelGGL((xprep_kernel<N2, XR, 512 * XR / N2>), grid, dim3(N2), 0, stream, *p);
-    else
-        hipLaunchKernelGGL((xprep_kernel<1024, XR, XR>), grid, dim3(1024), 0, stream, *p);
+    if (p->K <= 2048)
+        hipLaunchKernelGGL((xprep_kernel<64 * XR, XR>), grid, dim3(64 * XR), 0, stream, *p);
+    else if (p->K <= 4096)
+        hipLaunchKernelGGL((xprep_kernel<128 * XR, XR>), grid, dim3(128 * XR), 0, stream, *p);
+    else    /* at most 1024 threads: 4 rows */
+        hipLaunchKernelGGL((xprep_kernel<1024, 4>), dim3((p->M + 3) / 4), dim3(1024), 0, stream, *p);
 }
 }  // namespace
 
@@ -694,11 +775,11 @@ extern "C" hipError_t q35_mlx4_xprep(const Q35Mlx4Xprep *p, hipStream_t stream) 
      *   M = 2048: 10.3 |  7.5 |  8.2;  19.1 | 12.7 | 11.6
      *   M = 4096: 19.4 | 12.6 | 11.6;  36.7 | 23.0 | 21.5 */
     if (p->M <= 256)
-        launch_xprep<2, 512, 1024>(p, stream);
+        launch_xprep<2>(p, stream);
     else if (p->M <= 2048)
-        launch_xprep<4, 512, 1024>(p, stream);
+        launch_xprep<4>(p, stream);
     else
-        launch_xprep<8, 512, 512>(p, stream);
+        launch_xprep<8>(p, stream);
     return hipGetLastError();
 }
 
@@ -720,11 +801,10 @@ extern "C" hipError_t q35_mlx4_gemm(const Q35Mlx4Gemm *p, hipStream_t stream) {
     tiles *= p->Mpad / MT;
     if (tiles >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
     const int few = few_tokens(p);
-    if (few == 1) return launch_few<1, 1, 8>(p, stream);
-    if (few == 2) return launch_few<1, 2, 8>(p, stream);
-    if (few == 3) return launch_few<2, 2, 8>(p, stream);
-    if (few == 4) return launch_few<2, 2, 4>(p, stream);
-    hipLaunchKernelGGL(gemm_kernel, dim3((unsigned)tiles), dim3(NT), 0, stream, *p);
+    if (few == 1) return launch_few<1, 1>(p, stream);
+    if (few == 2) return launch_few<1, 2>(p, stream);
+    if (few == 3) return launch_few<2, 2>(p, stream);
+    hipLaunchKernelGGL(gemm_kernel, dim3((unsigned)tiles), dim3(64 * NW), 0, stream, *p);
     return hipGetLastError();
 }
 

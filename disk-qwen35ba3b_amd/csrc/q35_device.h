@@ -13,6 +13,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4_t;
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2_t;
+typedef __attribute__((ext_vector_type(6))) unsigned u32x6_t;
+typedef __attribute__((ext_vector_type(32))) float f32x32_t;
 
 /* A pointer every lane holds the same value of, moved to scalar registers.
  * A buffer resource must be uniform; built from an address the compiler
@@ -142,23 +144,51 @@ __device__ __forceinline__ T q35_half_sum(T v) {
 }
 
 /* The chunk GEMM's tiled X operand (written by its X prep and by the
- * delta-rule prefill's gated norm): x[m][k] of rows K wide as fp16 hi and
- * lo (x - hi), per 64-row tile and 64-column group g (G = K / 64) a 16 KB
- * block, hi then lo, each the group's MFMA operands as they are read: word
- * v = k / 8 of the row, with v % 8 = 4 h + ks, is the operand of lane half h
- * in k-step ks, so the granule of (row r, word v) is ((r / 32) 4 + ks) 64 +
- * 32 h + r % 32: one operand of a wave is 1 KB in lane order, read from LDS
- * without bank conflicts and from memory as whole lines.  Half j of a
- * granule holds k % 8 = q35_xw_perm(j), the order 0,4,1,5,2,6,3,7 in which a
- * nibble word's values become fp16 pairs. */
-constexpr int Q35_XW_ROWS = 64;
-constexpr int Q35_XW_BLK = Q35_XW_ROWS * 128;
-__device__ __forceinline__ int q35_xw_perm(int j) { return (j >> 1) + 4 * (j & 1); }
-/* byte offset of the hi granule of word v of row m (lo: + Q35_XW_BLK) */
-__device__ __forceinline__ size_t q35_xw_granule(int m, int v, int G) {
-    const int r = m & (Q35_XW_ROWS - 1), j = v & 7;
-    return ((size_t)(m / Q35_XW_ROWS) * G + (v >> 3)) * (2 * Q35_XW_BLK) +
-           ((((r >> 5) * 4 + (j & 3)) * 64 + (j >> 2) * 32 + (r & 31)) << 4);
+ * delta-rule prefill's gated norm).  The 32 columns a lane of an MFMA holds
+ * (row r % 32, columns 32 h .. of a 64-column group, lane 32 h + r % 32) are
+ * five fp6 (e2m3) digits to the base 32 under one exponent: digit 0 is x
+ * rounded at 2^(E0 - 127), the block's largest value being 2 to 4 of those,
+ * and digit d what the digits before it leave, at 2^(E0 - 5 d - 127).  A
+ * remainder is at most 1/32 of 4 units, so each digit stays within 4, and
+ * the five carry x to 2^-24 of the block's largest value (2^-25 for most).
+ * Per (32 rows, group; G = K / 64 groups a row) a block of 8 KB: per digit
+ * 64 lanes x the first 16 bytes of a lane's 24, then 64 x the other 8, and
+ * at Q35_XW_EXP 64 x 8 bytes, the digits' five exponent bytes.  Field
+ * f of a lane is column (f >> 1) + 16 (f & 1), the order in which the
+ * conversion interleaves its two 16-value operands. */
+constexpr int Q35_XW_ROWS = 64;            /* rows are allocated in tiles of this */
+constexpr int Q35_XW_BLK = 8192, Q35_XW_DIGITS = 5, Q35_XW_DIG = 1536;
+constexpr int Q35_XW_EXP = Q35_XW_DIGITS * Q35_XW_DIG;
+__device__ __forceinline__ int q35_xw_col(int f) { return (f >> 1) + 16 * (f & 1); }
+/* byte offset of the block of row m, group g */
+__device__ __forceinline__ size_t q35_xw_block(int m, int g, int G) {
+    return ((size_t)(m >> 5) * G + g) * Q35_XW_BLK;
+}
+/* a: columns 0..15 of the lane's 32, b: 16..31, sum: their sum, max: their
+ * largest magnitude.  A NaN or infinity (the sum is neither finite nor
+ * ordered then) gives the exponent 255, with which the MFMA returns NaN. */
+__device__ __forceinline__ void q35_xw_store(uint8_t *blk, int lane, f32x16_t a, f32x16_t b, float sum,
+                                             float max) {
+    const int e0 = ::max((int)(__float_as_uint(max) >> 23) - 1, 21);
+#pragma unroll
+    for (int d = 0; d < Q35_XW_DIGITS; d++) {
+        const float unit = __uint_as_float((uint32_t)(e0 - 5 * d) << 23);
+        const u32x6_t c = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, b, unit);
+        uint8_t *dst = blk + d * Q35_XW_DIG;
+        *reinterpret_cast<u32x4_t *>(dst + 16 * lane) = u32x4_t{c[0], c[1], c[2], c[3]};
+        *reinterpret_cast<u32x2_t *>(dst + 1024 + 8 * lane) = u32x2_t{c[4], c[5]};
+        if (d + 1 < Q35_XW_DIGITS) {
+            const f32x32_t r = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(c, unit);
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                a[i] -= r[2 * i];
+                b[i] -= r[2 * i + 1];
+            }
+        }
+    }
+    u32x2_t ex = {(uint32_t)e0 * 0x01010101u - 0x0f0a0500u, (uint32_t)e0 - 20u};
+    if (!(fabsf(sum) < INFINITY)) ex = u32x2_t{~0u, ~0u};
+    *reinterpret_cast<u32x2_t *>(blk + Q35_XW_EXP + 8 * lane) = ex;
 }
 
 /* Direct-to-LDS loads (buffer_load ... lds): lane l's 16 (dma16) or 4

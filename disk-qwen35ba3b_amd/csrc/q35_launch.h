@@ -185,19 +185,19 @@ hipError_t q35_mlx4_matvec(const Q35Mlx4 *p, int njobs, hipStream_t stream);
 
 /* ---- MLX 4-bit projections of a prefill chunk on MFMA (mlx4_gemm.hip) ----
  * Y[M][N] = X[M][K] W^T for [N x K] 4-bit weights, K % 64 == 0.  X goes
- * through q35_mlx4_xprep first (optional RMSNorm, fp16 hi / lo in word
- * order, tiled per 64 rows and group; group sums); the weight's scales /
- * biases through q35_mlx4_sb once ((16 s, b - 16 s) per group and row). */
+ * through q35_mlx4_xprep first (optional RMSNorm, fp6 digits in operand
+ * order; group sums); the weight's scales / biases through q35_mlx4_sb and
+ * its words through q35_mlx4_wt once. */
 typedef struct Q35Mlx4Xprep {
     const float *x;                /* [M][ldx] */
     const uint16_t *norm_w;        /* [K] or NULL */
-    uint16_t *xw;                  /* Mpad * K * 2 halfs: hi / lo blocks per (64-row tile, group) */
+    uint16_t *xw;                  /* Mpad * K * 4 bytes: blocks per (32 rows, group), q35_device.h */
     float *xsum;                   /* [K/64][Mpad] */
     int M, Mpad, K, ldx;
     int *status;                   /* Q35_STATUS_GEMM_F16, or NULL */
 } Q35Mlx4Xprep;
 typedef struct Q35Mlx4SB {
-    float s, b;                    /* 16 scale, bias - 16 scale */
+    uint32_t w[2];                 /* 8 bytes a (group, row): [G][npad] fp32 scales, then BF16 biases */
 } Q35Mlx4SB;
 #define Q35_GEMM_MAX_JOBS 4
 typedef struct Q35Mlx4GemmJob {

@@ -340,7 +340,7 @@ int ds4f_hip_attn_step_async(int L, int token, float *state, void *stream);
  * stream: the whole of ds4f_attn_gqa_chunk (src/attn_qwen.c:1145-1252) or
  * ds4f_attn_linear_chunk (:977-1135), as src/main.c:604-660 calls them per
  * layer: the tokens' input_layernorm, the batched MLX 4-bit projections
- * (ds4f_mlx4_matvec_batch, src/kernels.c:581-619, here one fp16-MFMA GEMM
+ * (ds4f_mlx4_matvec_batch, src/kernels.c:581-619, here one fp6-MFMA GEMM
  * launch for all of a layer's projections), the layer's prefill core, the
  * batched output projection and the residual adds.  states holds B
  * pointers to the tokens' hidden states [hidden], updated in place.  The
@@ -358,9 +358,10 @@ int ds4f_gpu_attn_chunk(int L, int t0, int B, float *const *states);
  * that B (at any t0) allocates. */
 int ds4f_hip_attn_chunk_async(int L, int t0, int B, float *states, void *stream);
 
-/* The prefill paths compute with fp16 operands (the GQA prefill's q, k, v
- * and the chunk GEMM's X), which hold magnitudes below 65520; the
- * reference is fp32 throughout (src/attn_qwen.c:328-386, :1222-1231).
+/* The GQA prefill computes with fp16 operands (q, k, v), which hold
+ * magnitudes below 65520, and the chunk GEMM's X is checked against the same
+ * limit; the reference is fp32 throughout (src/attn_qwen.c:328-386,
+ * :1222-1231).
  * Their kernels set bits of a status word when a value is out of that
  * range: 1 = a GQA prefill operand, 2 = a chunk GEMM X operand.  The host
  * entries ds4f_gpu_gqa_prefill and ds4f_gpu_attn_chunk clear the word
