@@ -194,6 +194,100 @@ __device__ __forceinline__ void chunk_rows_load(ChunkRows &R, const Q35LinPrefil
     }
 }
 
+/* the chunk-local cumulative log-decay of value head h over the 64 lanes'
+ * tokens, into LDS and (out) the chunk's gate vector */
+__device__ __forceinline__ void decay_vectors(const Q35LinPrefill &p, double *sG, float *sBeta, int c, int h,
+                                              int lane, float g, float beta, bool out) {
+    double G = g;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(G, off);
+        if (lane >= off) G += o;
+    }
+    sG[lane] = G;
+    sBeta[lane] = beta;
+    if (!out) return;
+    const double Gc = __shfl(G, 63);
+    float *gv = p.gvec + ((size_t)c * p.v_heads + h) * Q35_LIN_GVEC;
+    gv[lane] = (float)exp(G);
+    gv[C + lane] = (float)exp(Gc - G);
+    gv[2 * C + lane] = beta;
+    if (lane == 0) gv[3 * C] = (float)exp(Gc);
+}
+
+/* T = (I + A)^-1 of both value heads of key head kh from the M blocks in MB
+ * (chunk_kernel), and out; ends with T still being read from TB */
+__device__ __forceinline__ void invert_blocks(const Q35LinPrefill &p, float *MB, float *TB, float *UD, int c,
+                                              int kh, int w, int t) {
+    const int VH = p.v_heads, lane = t & 63, l16 = lane & 15, lq = lane >> 4;
+            /* diagonal blocks: wave w inverts block a = w of both value heads,
+             * column kc of U_aa on lane kc (+16 for head 1; lanes 32-63 repeat
+             * lanes 0-31 and do not write) */
+            {
+                const int a = w, v = (lane >> 4) & 1, kc = lane & 15;
+                const float *Md = MB + (v * 10 + blk_q(a, a)) * BLK;
+                float u[16];
+    #pragma unroll
+                for (int s = 15; s >= 0; s--) {
+                    float4 mrow[4];
+    #pragma unroll
+                    for (int q = 0; q < 4; q++) mrow[q] = *reinterpret_cast<const float4 *>(&Md[s * BS + 4 * q]);
+                    float acc = s == kc ? 1.0f : 0.0f;
+    #pragma unroll
+                    for (int r = s + 1; r < 16; r++) acc = fmaf(-el(mrow[r >> 2], r & 3), u[r], acc);
+                    u[s] = acc;
+                }
+                if (lane < 32) {
+                    float *Td = TB + (v * 10 + blk_q(a, a)) * BLK + kc * BS;     /* T_aa row kc */
+    #pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        *reinterpret_cast<float4 *>(&Td[4 * q]) = make_float4(u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]);
+                    float *Ud = UD + (v * 4 + a) * BLK;
+    #pragma unroll
+                    for (int s = 0; s < 16; s++) Ud[s * BS + kc] = u[s];
+                }
+            }
+            q35_lds_barrier();
+
+            /* off-diagonal blocks by distance d = b - a: jobs (head v, block a),
+             * dealt round-robin over the waves; each is two 16x16x16 products */
+    #pragma unroll
+            for (int d = 1; d < 4; d++) {
+                for (int j = w; j < 2 * (4 - d); j += 4) {
+                    const int v = j / (4 - d), a = j % (4 - d), b = a + d;
+                    f32x4_t wacc = {0.f, 0.f, 0.f, 0.f};
+                    for (int cb = a + 1; cb <= b; cb++) {
+                        /* X = M_ac row-major; Y = U_cb, read as its transpose T_bc */
+                        const float4 xa = *reinterpret_cast<const float4 *>(&MB[(v * 10 + blk_q(a, cb)) * BLK + l16 * BS + 4 * lq]);
+                        const float4 yb = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(cb, b)) * BLK + l16 * BS + 4 * lq]);
+    #pragma unroll
+                        for (int e = 0; e < 4; e++) wacc = mfma4(el(xa, e), el(yb, e), wacc);
+                    }
+                    /* T_ba = (-W^T) U_aa^T: this lane's W entries W[4lq+e][l16] are
+                     * X[l16][4lq+e] of -W^T as they stand; Y^T = U_aa row-major */
+                    const float4 ud = *reinterpret_cast<const float4 *>(&UD[(v * 4 + a) * BLK + l16 * BS + 4 * lq]);
+                    f32x4_t tb = {0.f, 0.f, 0.f, 0.f};
+    #pragma unroll
+                    for (int e = 0; e < 4; e++) tb = mfma4(-wacc[e], el(ud, e), tb);
+                    float *Tt = TB + (v * 10 + blk_q(a, b)) * BLK;
+    #pragma unroll
+                    for (int i = 0; i < 4; i++) Tt[(4 * lq + i) * BS + l16] = tb[i];
+                }
+                q35_lds_barrier();
+            }
+
+            /* T out: 2 heads x the 10 lower blocks x 16 rows x 4 float4, each wave
+             * instruction one whole 1 KB block */
+    #pragma unroll
+            for (int u = 0; u < 5; u++) {
+                const int idx = u * 256 + t, v = idx / 640, rem = idx % 640;
+                const int j = rem >> 6, r = (rem >> 2) & 15, q4 = rem & 3;
+                const int bb = j < 1 ? 0 : j < 3 ? 1 : j < 6 ? 2 : 3, ba = j - tri_idx(bb, 0);
+                const float4 o = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(ba, bb)) * BLK + r * BS + 4 * q4]);
+                *reinterpret_cast<float4 *>(p.T + ((size_t)c * VH + 2 * kh + v) * C * C + j * 256 + r * 16 + 4 * q4) = o;
+            }
+}
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_kernel(Q35LinPrefill p) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __builtin_assume(w >= 0 && w < 4);     /* 256 threads: tile n = w + 4k is K K^T for k < 2, Q K^T for k > 2 */
@@ -219,18 +313,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const int c = it % p.n_chunks, kh = it / p.n_chunks;
         const int b0 = c * C, nv = min(C, p.B - b0);
 
-        /* the conv ring: slot pos % 4 <- raw row of pos for the last min(B, 4)
-         * tokens, written by the last chunk's items (the conv kernel, which
-         * reads the ring, has finished) */
-        if (c == p.n_chunks - 1) {
-            const int nr = min(p.B, 4), n4 = rows / 4;
-            for (int i = kh * 256 + t; i < nr * n4; i += KH * 256) {
-                const int b = p.B - nr + i / n4, c4 = 4 * (i % n4);
-                *reinterpret_cast<float4 *>(p.ring + (size_t)((p.t0 + b) & 3) * rows + c4) =
-                    *reinterpret_cast<const float4 *>(p.qkv + (size_t)b * rows + c4);
-            }
-        }
-
         /* gates and the chunk-local cumulative log-decay of value head 2kh + w
          * (pads: g = beta = 0) */
         if (w < 2) {
@@ -241,20 +323,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 g = gb.x;
                 beta = gb.y;
             }
-            double G = g;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const double o = __shfl_up(G, off);
-                if (lane >= off) G += o;
-            }
-            sG[w][lane] = G;
-            sBeta[w][lane] = beta;
-            const double Gc = __shfl(G, 63);
-            float *gv = p.gvec + ((size_t)c * VH + h) * Q35_LIN_GVEC;
-            gv[lane] = (float)exp(G);
-            gv[C + lane] = (float)exp(Gc - G);
-            gv[2 * C + lane] = beta;
-            if (lane == 0) gv[3 * C] = (float)exp(Gc);
+            decay_vectors(p, sG[w], sBeta[w], c, h, lane, g, beta, true);
         }
         /* the item's K and Q rows into LDS (pad rows zero), then the next
          * item's requested into the same registers */
@@ -338,74 +407,156 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         q35_lds_barrier();
 
-        /* diagonal blocks: wave w inverts block a = w of both value heads,
-         * column kc of U_aa on lane kc (+16 for head 1; lanes 32-63 repeat
-         * lanes 0-31 and do not write) */
-        {
-            const int a = w, v = (lane >> 4) & 1, kc = lane & 15;
-            const float *Md = MB + (v * 10 + blk_q(a, a)) * BLK;
-            float u[16];
-#pragma unroll
-            for (int s = 15; s >= 0; s--) {
-                float4 mrow[4];
-#pragma unroll
-                for (int q = 0; q < 4; q++) mrow[q] = *reinterpret_cast<const float4 *>(&Md[s * BS + 4 * q]);
-                float acc = s == kc ? 1.0f : 0.0f;
-#pragma unroll
-                for (int r = s + 1; r < 16; r++) acc = fmaf(-el(mrow[r >> 2], r & 3), u[r], acc);
-                u[s] = acc;
-            }
-            if (lane < 32) {
-                float *Td = TB + (v * 10 + blk_q(a, a)) * BLK + kc * BS;     /* T_aa row kc */
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-                    *reinterpret_cast<float4 *>(&Td[4 * q]) = make_float4(u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]);
-                float *Ud = UD + (v * 4 + a) * BLK;
-#pragma unroll
-                for (int s = 0; s < 16; s++) Ud[s * BS + kc] = u[s];
-            }
-        }
-        q35_lds_barrier();
-
-        /* off-diagonal blocks by distance d = b - a: jobs (head v, block a),
-         * dealt round-robin over the waves; each is two 16x16x16 products */
-#pragma unroll
-        for (int d = 1; d < 4; d++) {
-            for (int j = w; j < 2 * (4 - d); j += 4) {
-                const int v = j / (4 - d), a = j % (4 - d), b = a + d;
-                f32x4_t wacc = {0.f, 0.f, 0.f, 0.f};
-                for (int cb = a + 1; cb <= b; cb++) {
-                    /* X = M_ac row-major; Y = U_cb, read as its transpose T_bc */
-                    const float4 xa = *reinterpret_cast<const float4 *>(&MB[(v * 10 + blk_q(a, cb)) * BLK + l16 * BS + 4 * lq]);
-                    const float4 yb = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(cb, b)) * BLK + l16 * BS + 4 * lq]);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) wacc = mfma4(el(xa, e), el(yb, e), wacc);
-                }
-                /* T_ba = (-W^T) U_aa^T: this lane's W entries W[4lq+e][l16] are
-                 * X[l16][4lq+e] of -W^T as they stand; Y^T = U_aa row-major */
-                const float4 ud = *reinterpret_cast<const float4 *>(&UD[(v * 4 + a) * BLK + l16 * BS + 4 * lq]);
-                f32x4_t tb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int e = 0; e < 4; e++) tb = mfma4(-wacc[e], el(ud, e), tb);
-                float *Tt = TB + (v * 10 + blk_q(a, b)) * BLK;
-#pragma unroll
-                for (int i = 0; i < 4; i++) Tt[(4 * lq + i) * BS + l16] = tb[i];
-            }
-            q35_lds_barrier();
-        }
-
-        /* T out: 2 heads x the 10 lower blocks x 16 rows x 4 float4, each wave
-         * instruction one whole 1 KB block */
-#pragma unroll
-        for (int u = 0; u < 5; u++) {
-            const int idx = u * 256 + t, v = idx / 640, rem = idx % 640;
-            const int j = rem >> 6, r = (rem >> 2) & 15, q4 = rem & 3;
-            const int bb = j < 1 ? 0 : j < 3 ? 1 : j < 6 ? 2 : 3, ba = j - tri_idx(bb, 0);
-            const float4 o = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(ba, bb)) * BLK + r * BS + 4 * q4]);
-            *reinterpret_cast<float4 *>(p.T + ((size_t)c * VH + 2 * kh + v) * C * C + j * 256 + r * 16 + 4 * q4) = o;
-        }
+        invert_blocks(p, MB, TB, UD, c, kh, w, t);
         q35_lds_barrier();                       /* T read out: the next item may overwrite the LDS */
     }
+}
+
+/* ---- the two kernels before the scan in one launch, for few chunks -------- *
+ * With few chunks conv_kernel and chunk_kernel are two short launches of
+ * which each waits out its own memory round trips, and chunk_kernel's WG
+ * count is 16 a chunk.  Here an item (chunk, key head) is three workgroups, each
+ * convolving the raw rows of the heads it needs (64 + 3 rows, all loads ahead
+ * of the first use; half-wave hw has tokens 8 hw .. + 7, 4 channels a lane):
+ * role 0 K -> K K^T, T, the gate vectors; role 1 Q and K -> Q K^T, Pm; role 2
+ * the two value heads.  K is convolved twice and the gates twice; nothing
+ * passes through memory between the two steps.  The arithmetic is conv_kernel's
+ * and chunk_kernel's, in their order: results are bit-identical. */
+__device__ __forceinline__ void conv_head(const Q35LinPrefill &p, int c, int grp, bool store, float *lds) {
+    const int t = threadIdx.x, hw = t >> 5, KH = p.k_heads, rows = 2 * KH * KD + p.v_heads * VD;
+    const int c0 = grp * KD + 4 * (t & 31), b0 = c * C, bb = b0 + 8 * hw;
+    const uint4 wa = *reinterpret_cast<const uint4 *>(p.conv_w + (size_t)c0 * 4);
+    const uint4 wb = *reinterpret_cast<const uint4 *>(p.conv_w + (size_t)c0 * 4 + 8);
+    const int r0 = max(b0 - 3, 0);
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+        q35_uniform_ptr(const_cast<float *>(p.qkv) + (size_t)r0 * rows), 0, min(p.B - r0, C + 3) * rows * 4,
+        Q35_BUF_DW3);
+    float4 xr[11];
+#pragma unroll
+    for (int k = 0; k < 11; k++) {
+        const int b = bb - 3 + k;
+        xr[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               rq, b >= 0 ? (uint32_t)(((b - r0) * rows + c0) * 4) : 0x80000000u, 0, 0));
+    }
+    if (c == 0) {                      /* the three rows before the batch: the ring */
+        const __amdgpu_buffer_rsrc_t rr =
+            __builtin_amdgcn_make_buffer_rsrc(q35_uniform_ptr(p.ring), 0, 4 * rows * 4, Q35_BUF_DW3);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const int pp = p.t0 - 3 + k;
+            const float4 x = __builtin_bit_cast(
+                float4, __builtin_amdgcn_raw_buffer_load_b128(
+                            rr, pp >= 0 ? (uint32_t)(((pp & 3) * rows + c0) * 4) : 0x80000000u, 0, 0));
+            if (hw == 0) xr[k] = x;
+        }
+    }
+    const uint2 wt[4] = {make_uint2(wa.x, wa.y), make_uint2(wa.z, wa.w), make_uint2(wb.x, wb.y),
+                         make_uint2(wb.z, wb.w)};
+    const float scale = grp < KH ? 1.0f / (float)KD : 1.0f / sqrtf((float)KD);
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int b = bb + j;
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float x[4] = {el(xr[j], e), el(xr[j + 1], e), el(xr[j + 2], e), el(xr[j + 3], e)};
+            y[e] = q35_conv_silu_fast(x, wt[e], p.t0 + b);
+        }
+        if (grp < 2 * KH) {
+#pragma clang fp contract(off)
+            float ss = y[0] * y[0] + y[1] * y[1] + y[2] * y[2] + y[3] * y[3];
+            ss = q35_half_sum(ss);
+            const float r = sqrtf(ss * (1.0f / (float)KD) + 1e-6f), ri = 1.0f / r;
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[e] = y[e] * ri * scale;
+        }
+        const bool live = b < p.B;
+        const float4 o = live ? make_float4(y[0], y[1], y[2], y[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if (store && live) *reinterpret_cast<float4 *>(p.post + (size_t)b * rows + c0) = o;
+        if (lds) *reinterpret_cast<float4 *>(&lds[sw128(8 * hw + j, 4 * (t & 31))]) = o;
+    }
+}
+
+__global__ __launch_bounds__(256) void chunk_few_kernel(Q35LinPrefill p) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __builtin_assume(w >= 0 && w < 4);
+    const int KH = p.k_heads, VH = p.v_heads, n_items = p.n_chunks * KH;
+    const int role = blockIdx.x / n_items, it = blockIdx.x % n_items;
+    const int c = it % p.n_chunks, kh = it / p.n_chunks;
+    const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, lq = lane >> 4;
+    __shared__ __align__(16) float sbuf[2 * C * KD];
+    __shared__ __align__(16) double sG[2][C];
+    __shared__ __align__(16) float sBeta[2][C];
+    float *sK = sbuf, *sQ = sbuf + C * KD;
+
+    if (role == 2) {
+        conv_head(p, c, 2 * KH + 2 * kh, true, nullptr);
+        conv_head(p, c, 2 * KH + 2 * kh + 1, true, nullptr);
+        return;
+    }
+    conv_head(p, c, KH + kh, role == 0, sK);
+    if (role == 1) conv_head(p, c, kh, true, sQ);
+    if (w < 2) {
+        const int h = 2 * kh + w, b = c * C + lane;
+        float g = 0.f, beta = 0.f;
+        if (b < p.B)
+            q35_lin_gates(p.a[(size_t)b * VH + h], p.b[(size_t)b * VH + h], p.A_log[h], p.dt_bias[h], &g, &beta);
+        decay_vectors(p, sG[w], sBeta[w], c, h, lane, g, beta, role == 0);
+    }
+    q35_lds_barrier();
+
+    /* the 10 lower 16x16 tiles of K K^T (role 0) or Q K^T, as chunk_kernel's */
+    const float *X = role == 0 ? sK : sQ;
+    f32x4_t res[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int m = w + 4 * k;
+        if (m >= 10) break;
+        const int tr = m < 1 ? 0 : m < 3 ? 1 : m < 6 ? 2 : 3;
+        const int tc = m - (tr * (tr + 1)) / 2;
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int blk = 0; blk < KD / 16; blk++) {
+            const float4 xa = *reinterpret_cast<const float4 *>(&X[sw128(16 * tr + l16, 16 * blk + 4 * lq)]);
+            const float4 yb = *reinterpret_cast<const float4 *>(&sK[sw128(16 * tc + l16, 16 * blk + 4 * lq)]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = mfma4(el(xa, e), el(yb, e), acc);
+        }
+        res[k] = acc;
+    }
+    q35_lds_barrier();                           /* K no longer read */
+    float *MB = sbuf, *TB = sbuf + 2 * 10 * BLK, *UD = sbuf + 4 * 10 * BLK;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int m = w + 4 * k;
+        if (m >= 10) break;
+        const int tr = m < 1 ? 0 : m < 3 ? 1 : m < 6 ? 2 : 3;
+        const int tc = m - (tr * (tr + 1)) / 2;
+        const int s = 16 * tc + l16, r0 = 16 * tr + 4 * lq;
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            const double gs = sG[v][s];
+            float o[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int r = r0 + i;
+                const float dec = __expf((float)(sG[v][r] - gs));
+                const float av = sBeta[v][r] * dec * res[k][i], pv = dec * res[k][i];
+                o[i] = role == 0 ? (s < r ? av : 0.0f) : (s <= r ? pv : 0.0f);
+            }
+            if (role == 0) {
+                *reinterpret_cast<float4 *>(&MB[(v * 10 + blk_q(tc, tr)) * BLK + l16 * BS + 4 * lq]) =
+                    make_float4(o[0], o[1], o[2], o[3]);
+            } else {
+                float *Pm = p.Pm + ((size_t)c * VH + 2 * kh + v) * C * C + tri_idx(tr, tc) * 256;
+#pragma unroll
+                for (int i = 0; i < 4; i++) Pm[(4 * lq + i) * 16 + l16] = o[i];
+            }
+        }
+    }
+    if (role == 1) return;
+    q35_lds_barrier();
+    invert_blocks(p, MB, TB, UD, c, kh, w, t);
 }
 
 /* ---- 4. sequential scan over chunks per (value head, 16-column block) ---- *
@@ -743,6 +894,16 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_kernel(Q35LinPrefill p) {
 
     /* ---- compute waves ---- */
     const int w = wave, lane = t & 63;
+    /* the conv ring: slot pos % 4 <- raw row of pos for the last min(B, 4)
+     * tokens (the kernels that read the ring have finished) */
+    {
+        const int nr = min(p.B, 4), n4 = g.rows / 4;
+        for (int i = n * 256 + t; i < nr * n4; i += (int)gridDim.x * 256) {
+            const int b = p.B - nr + i / n4, c4 = 4 * (i % n4);
+            *reinterpret_cast<float4 *>(p.ring + (size_t)((p.t0 + b) & 3) * g.rows + c4) =
+                *reinterpret_cast<const float4 *>(p.qkv + (size_t)b * g.rows + c4);
+        }
+    }
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int idx = u * 256 + t, jj = idx >> 5, i4 = (idx & 31) * 4;
@@ -777,6 +938,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_kernel(Q35LinPrefill p) {
  * A lane of that operand is 32 columns of a row, so the wave's rows pass
  * through its own LDS area and lane (token l % TT, quarter l / TT of the
  * head) stores the digits, 16 TT consecutive bytes a quarter. */
+constexpr int FEW_TOKENS = 1024;
 constexpr int GTT = 4;
 template <int TT, bool XW>
 __global__ __launch_bounds__(256) void gnorm_kernel(Q35LinPrefill p) {
@@ -864,10 +1026,14 @@ extern "C" hipError_t q35_lin_prefill(const Q35LinPrefill *pin, hipStream_t stre
         return hipErrorInvalidValue;
     /* checked before any launch: the kernels advance the ring and state in place */
     if (p.xw && (p.mpad < p.B || p.mpad % Q35_XW_ROWS != 0 || !p.xsum)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(conv_kernel, dim3(rows / 1024, (p.B + CT - 1) / CT), dim3(256), 0, stream, p);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(chunk_kernel, dim3(min(p.n_chunks * p.k_heads, CHUNK_GRID)), dim3(256), 0, stream, p);
+    hipError_t e;
+    if (p.B <= FEW_TOKENS) {
+        hipLaunchKernelGGL(chunk_few_kernel, dim3(3 * p.n_chunks * p.k_heads), dim3(256), 0, stream, p);
+    } else {
+        hipLaunchKernelGGL(conv_kernel, dim3(rows / 1024, (p.B + CT - 1) / CT), dim3(256), 0, stream, p);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(chunk_kernel, dim3(min(p.n_chunks * p.k_heads, CHUNK_GRID)), dim3(256), 0, stream, p);
+    }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(scan_kernel, dim3(p.v_heads * (VD / 16)), dim3(SCAN_THREADS), 0, stream, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
