@@ -457,9 +457,9 @@ int ds4f_hip_gqa_prefill_async(int L, int t0, int B, const float *q_gate, const 
     size_t kb, vb, kr, vr;
     q35_gqa_prefill_ws_bytes(t0, B, P.g.n_kv_heads, &kb, &vb);
     q35_gqa_prefill_ws_bytes(0, P.g.max_tokens, P.g.n_kv_heads, &kr, &vr);
-    size_t mb;
-    const size_t pb = q35_gqa_prefill_part_bytes(&mb);
-    if (ensure_ws(kr + vr + pb + mb) != 0) return -1;
+    size_t mb, qb;
+    const size_t pb = q35_gqa_prefill_part_bytes(&mb, &qb);
+    if (ensure_ws(kr + vr + pb + mb + qb) != 0) return -1;
     Q35GqaPrefill p;
     memset(&p, 0, sizeof p);
     p.q_gate = q_gate;
@@ -474,6 +474,7 @@ int ds4f_hip_gqa_prefill_async(int L, int t0, int B, const float *q_gate, const 
     p.vw = (uint16_t *)((char *)P.d_ws + kb);
     p.part = (float *)((char *)P.d_ws + kr + vr);
     p.part_ml = (float *)((char *)P.d_ws + kr + vr + pb);
+    p.qw = (uint16_t *)((char *)P.d_ws + kr + vr + pb + mb);
     p.attn_out = attn_out;
     p.k_post = k_post;
     p.t0 = t0;

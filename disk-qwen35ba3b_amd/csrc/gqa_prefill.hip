@@ -131,6 +131,65 @@ __device__ __forceinline__ void prep_rows(const Q35GqaPrefill &p, int bx) {
     }
 }
 
+/* halfs offset of the MFMA operand of q block qb, wave wg of its four, k-step
+ * ks, in the q workspace: 64 lanes x 8 halfs, lane (col, h) as load_q's */
+__device__ __forceinline__ size_t qw_index(int g, int nqb, int qb, int wg, int ks) {
+    return ((((size_t)g * nqb + qb) * 4 + wg) * 16 + ks) * 64 * 8;
+}
+
+/* q of the new tokens as the attention kernel's operand, two heads a wave:
+ * load_q's norm and rotation, a head's 256 dims over the lanes.  In the
+ * attention kernel a load takes 64 bytes of each of 32 rows, which keeps a
+ * CU's address unit busy for 17,000 cycles; where a block's keys are many
+ * spans, every one of its workgroups would do that. */
+__device__ __forceinline__ void prep_q(const Q35GqaPrefill &p, int bx) {
+    const int lane = threadIdx.x & 63, d0 = lane * 4, w = threadIdx.x >> 6;
+    const int row0 = 8 * bx + 2 * w, b = row0 / p.heads, pos = p.t0 + b;   /* heads is even */
+    if (b >= p.B) return;
+    const float *rope = p.rope + (size_t)pos * RD;
+    float4 rc = make_float4(1.f, 1.f, 1.f, 1.f), rs = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (lane < RD / 4) {
+        rc = *reinterpret_cast<const float4 *>(rope + (d0 & (RD / 2 - 1)));
+        rs = *reinterpret_cast<const float4 *>(rope + RD / 2 + (d0 & (RD / 2 - 1)));
+    }
+    const uint2 wq = *reinterpret_cast<const uint2 *>(p.qn_w + d0);
+    float4 x[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+        x[u] = *reinterpret_cast<const float4 *>(p.q_gate + (size_t)(row0 + u) * 2 * D + d0);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+#pragma clang fp contract(off)
+        const int head = row0 % p.heads + u, g = head / G, hl = head % G;
+        double ss = (double)x[u].x * x[u].x + (double)x[u].y * x[u].y + (double)x[u].z * x[u].z +
+                    (double)x[u].w * x[u].w;
+        ss = q35_wave_sum(ss);
+        const float r = sqrtf((float)(ss / (double)D) + 1e-6f), ri = 1.0f / r;
+        float v[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+        const float cc[4] = {rc.x, rc.y, rc.z, rc.w}, sn[4] = {rs.x, rs.y, rs.z, rs.w};
+        uint16_t o[4];
+        bool over = false;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            v[e] = v[e] * ri * q35_bf2f((uint16_t)((e < 2 ? wq.x : wq.y) >> (16 * (e & 1))));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float pr = q35_xor8(v[e]);
+            float y = v[e];
+            if (lane < RD / 8)
+                y = v[e] * cc[e] - pr * sn[e];       /* x0*c - x1*s */
+            else if (lane < RD / 4)
+                y = pr * sn[e] + v[e] * cc[e];       /* x0*s + x1*c */
+            over = over || q35_f16_over(y);
+            o[e] = f16_bits(y);
+        }
+        q35_f16_guard(p.status, Q35_STATUS_GQA_F16, over);
+        const int col = (hl & 1) * 16 + (b & 15), h = (d0 >> 3) & 1;
+        uint16_t *dst = p.qw + qw_index(g, p.nqb, b >> 4, hl >> 1, d0 >> 4) + (32 * h + col) * 8 + (d0 & 4);
+        *reinterpret_cast<uint2 *>(dst) = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+    }
+}
+
 /* v of the new tokens -> the fp16 value workspace and the bf16 cache,
  * both dim-major ([dim][keys]).  One workgroup per (32-key block, kv head)
  * transposes the block's rows through LDS; a lane then stores 8 keys of
@@ -290,9 +349,9 @@ __device__ __forceinline__ void prefix_rows(const Q35GqaPrefill &p, int n_rows, 
  * elements; as separate launches the dispatch gaps and the smaller kernels'
  * tails cost about as much as the work): blocks [0, nk) prep_rows, the next
  * nvb * kv_heads blocks vprep_block, then t0 / 32 * kv_heads of prefix_tile,
- * the rest prefix_rows.  Every branch is block-uniform, so vprep_block's
+ * nq of prep_q, the rest prefix_rows.  Every branch is block-uniform, so vprep_block's
  * barrier sees all of its block's threads. */
-__global__ __launch_bounds__(256) void prep_kernel(Q35GqaPrefill p, int nvb, int n_rows) {
+__global__ __launch_bounds__(256) void prep_kernel(Q35GqaPrefill p, int nvb, int n_rows, int nq) {
     const int nk = (p.B + 3) / 4, nv = nvb * p.kv_heads, nt = p.t0 >> 5;
     int bx = (int)blockIdx.x;
     if (bx < nk) {
@@ -301,8 +360,10 @@ __global__ __launch_bounds__(256) void prep_kernel(Q35GqaPrefill p, int nvb, int
         vprep_block(p, bx % nvb, bx / nvb);
     } else if ((bx -= nv) < nt * p.kv_heads) {
         prefix_tile(p, bx % nt, bx / nt);
+    } else if ((bx -= nt * p.kv_heads) < nq) {
+        prep_q(p, bx);
     } else {
-        prefix_rows(p, n_rows, bx - nt * p.kv_heads);
+        prefix_rows(p, n_rows, bx - nq);
     }
 }
 
@@ -504,7 +565,7 @@ __device__ __forceinline__ void load_q(const Q35GqaPrefill &p, int g, int qb, in
  * of them and group B the rest, as in the long block above; a block of
  * several spans leaves its merged (max, sum, O), fp32, to
  * span_merge_kernel. */
-template <bool SPLIT>
+template <bool SPLIT, bool QW>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kernel(Q35GqaPrefill p) {
     /* 1-D grid over (pair, kv head).  Workgroups go to the 8 XCDs in turn
      * (id mod 8); with the pair count a multiple of 4, XCDs 0-3 take kv
@@ -703,13 +764,24 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kern
         sched_reads_ahead<2>();   /* PV: two reads ahead (four: +5 us a call at 4096 tokens) */
     };
 
+    /* q of block qb: made here, or (QW) read from the workspace */
+    auto get_q = [&](int qb) {
+        if constexpr (QW) {
+#pragma unroll
+            for (int ks = 0; ks < 16; ks++)
+                qop[ks] = *reinterpret_cast<const f16x8_t *>(p.qw + qw_index(g, p.nqb, qb, wg, ks) + lane * 8);
+        } else {
+            load_q(p, g, qb, hl, col, h, qop);
+        }
+    };
     reset();
     f32x16_t s;
     const Dma2 dnone = dma2(0, 0, 0, 0, 0, 0);
     if (grp == 0) {
-        load_q(p, g, qL, hl, col, h, qop);
+        if constexpr (!QW) get_q(qL);
         stage_part(0, 0, c0);
         stage_part(0, 1, c0);
+        if constexpr (QW) get_q(qL);             /* the first tiles are on their way */
         wait_dma();
         q35_lds_barrier();
         for (int it = 0; it < nA; it++) {
@@ -724,8 +796,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kern
         }
     } else {
         if (nB > 0) {
-            load_q(p, g, block_b(0), hl, col, h, qop);
+            if constexpr (!QW) get_q(block_b(0));
             stage_part(0, 0, tile_b(0));
+            if constexpr (QW) get_q(block_b(0));
         }
         wait_dma();
         q35_lds_barrier();
@@ -746,7 +819,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void attn_kern
                      * block's tail next */
                     store_rows(p, g, qS, hl, col, h, l_run, acc);
                     reset();
-                    load_q(p, g, qL, hl, col, h, qop);
+                    get_q(qL);
                     /* all of this wave's loads done: the compiler then
                      * places no load-count waits for q on the common
                      * path, where they would also wait for staging loads */
@@ -916,16 +989,20 @@ __global__ __launch_bounds__(256) void span_merge_kernel(Q35GqaPrefill p) {
  *     its two blocks in turn, 10 more;
  *   - partials cost 1 for the merge launch and 0.07 a span for the 256 KB
  *     its two kv heads write and read (so spans of a few tiles lose: 64
- *     tokens at 4032 in 8 / 16 / 32 spans 40.9 / 36.7 / 39.1 us, whole op);
+ *     tokens at 4032 in 8 / 16 / 32 spans 31.3 / 27.7 / 31.1 us, whole op);
  *   - past 256 workgroups, blocks go longest first: the end is the average
  *     load, half of the shortest block and 14 for the uneven last round.
  * The pair form is left for more than 128 blocks that start near position
  * 0, whose lengths differ most (at 0, pairs / one span a block: 4096 tokens
- * 184 / 191 us, 3500 132 / 137; but 2048 90 / 79, 64 32.3 / 26.8, 5000 335 /
+ * 184 / 191 us, 3500 132 / 137; but 2048 90 / 79, 64 32.2 / 18.0, 5000 335 /
  * 275, whose pairs need a second round; 2500 at 2000 191 / 186).  The
- * 500-token prefill at 12345 took 582 us with pairs (32 workgroups) and 131
- * in 4 spans, 64 tokens at 32000 1318 and 79 in 32. */
+ * 500-token prefill at 12345 took 544 us with pairs (32 workgroups) and takes
+ * 128 in 4 spans, 64 tokens at 32000 1299 and 71 in 32. */
 constexpr int CUS = 256;
+/* the q workspace holds this many tokens (us a call, q made in the attention
+ * kernel -> in the set-up: 64 at 0 26.8 -> 18.1, 64 at 4032 36.7 -> 27.8, 1000
+ * at 0 51.4 -> 47.8; the gain falls with the tokens, whose q the set-up writes and reads back) */
+constexpr int QW_TOKENS = 1024;
 int spans_for(int t0, int B, int *span_tiles) {
     const int nqb = (B + 15) / 16, n1 = (min(t0 + 16, t0 + B) + 31) / 32, n2 = (t0 + B + 31) / 32;
     double best = ((nqb + 1) / 2 * 2 + CUS - 1) / CUS * ((n1 + n2 + 1) / 2 + 16.0);
@@ -953,8 +1030,9 @@ extern "C" void q35_gqa_prefill_ws_bytes(int t0, int B, int kv_heads, size_t *kw
     *vw = *kw;
 }
 
-extern "C" size_t q35_gqa_prefill_part_bytes(size_t *ml) {
+extern "C" size_t q35_gqa_prefill_part_bytes(size_t *ml, size_t *qw) {
     *ml = (size_t)CUS * 128 * 2 * 8;
+    *qw = (size_t)QW_TOKENS * 2 * G * D * 2;
     return (size_t)CUS * 128 * D * 4;
 }
 
@@ -967,18 +1045,24 @@ extern "C" hipError_t q35_gqa_prefill(const Q35GqaPrefill *pin, hipStream_t stre
      * those leave: the prefix's last, partial tile and the key padding */
     const int nvb = ((p.t0 + p.B - 1) >> 5) - (p.t0 >> 5) + 1;
     const int n_rows = (p.t0 & 31) + (p.kbt * 32 - (p.t0 + p.B));
-    const int64_t nblk = (p.B + 3) / 4 + (int64_t)nvb * p.kv_heads + (int64_t)(p.t0 >> 5) * p.kv_heads +
+    p.spans = spans_for(p.t0, p.B, &p.span_tiles);
+    const bool qw = p.spans > 0 && p.B <= QW_TOKENS;
+    const int nq = qw ? (p.B * p.heads + 7) / 8 : 0;
+    const int64_t nblk = nq + (p.B + 3) / 4 + (int64_t)nvb * p.kv_heads + (int64_t)(p.t0 >> 5) * p.kv_heads +
                          ((int64_t)p.kv_heads * n_rows * D + 255) / 256;
     if (nblk > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(prep_kernel, dim3((unsigned)nblk), dim3(256), 0, stream, p, nvb, n_rows);
+    hipLaunchKernelGGL(prep_kernel, dim3((unsigned)nblk), dim3(256), 0, stream, p, nvb, n_rows, nq);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    p.spans = spans_for(p.t0, p.B, &p.span_tiles);
     if (p.spans == 0) {
-        hipLaunchKernelGGL(attn_kernel<false>, dim3((p.nqb + 1) / 2 * p.kv_heads), dim3(512), 0, stream, p);
+        hipLaunchKernelGGL((attn_kernel<false, false>), dim3((p.nqb + 1) / 2 * p.kv_heads), dim3(512), 0, stream, p);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(attn_kernel<true>, dim3(p.nqb * p.spans * p.kv_heads), dim3(512), 0, stream, p);
+    const dim3 grid(p.nqb * p.spans * p.kv_heads);
+    if (qw)
+        hipLaunchKernelGGL((attn_kernel<true, true>), grid, dim3(512), 0, stream, p);
+    else
+        hipLaunchKernelGGL((attn_kernel<true, false>), grid, dim3(512), 0, stream, p);
     e = hipGetLastError();
     if (e != hipSuccess || p.spans == 1) return e;
     hipLaunchKernelGGL(span_merge_kernel, dim3(p.nqb * p.kv_heads * MERGE_SPLIT), dim3(256), 0, stream, p);

@@ -118,6 +118,7 @@ typedef struct Q35GqaPrefill {
     uint16_t *kt, *vt;             /* this layer's K / V cache tiles */
     uint16_t *kw, *vw;             /* fp16 workspaces */
     float *part, *part_ml;         /* partials of split q blocks */
+    uint16_t *qw;                  /* fp16 q operands of short calls */
     float *attn_out;               /* [B][H][D] */
     float *k_post;                 /* optional [B][KVH][D] */
     int t0, B, t_tiles, heads, kv_heads;
@@ -125,8 +126,9 @@ typedef struct Q35GqaPrefill {
     int *status;                   /* Q35_STATUS_GQA_F16, or NULL */
 } Q35GqaPrefill;
 void q35_gqa_prefill_ws_bytes(int t0, int B, int kv_heads, size_t *kw, size_t *vw);
-/* bytes of part and (ml) part_ml: 256 spans of 128 columns, whatever t0 and B */
-size_t q35_gqa_prefill_part_bytes(size_t *ml);
+/* bytes of part, part_ml and qw, whatever t0 and B: 256 spans of 128 columns,
+ * the q of 1024 tokens */
+size_t q35_gqa_prefill_part_bytes(size_t *ml, size_t *qw);
 hipError_t q35_gqa_prefill(const Q35GqaPrefill *p, hipStream_t stream);
 
 /* ---- state movement between host row layouts and device layouts ---- */
