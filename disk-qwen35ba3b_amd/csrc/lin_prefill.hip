@@ -217,75 +217,77 @@ __device__ __forceinline__ void decay_vectors(const Q35LinPrefill &p, double *sG
 
 /* T = (I + A)^-1 of both value heads of key head kh from the M blocks in MB
  * (chunk_kernel), and out; ends with T still being read from TB */
+template <int NW>
 __device__ __forceinline__ void invert_blocks(const Q35LinPrefill &p, float *MB, float *TB, float *UD, int c,
                                               int kh, int w, int t) {
     const int VH = p.v_heads, lane = t & 63, l16 = lane & 15, lq = lane >> 4;
-            /* diagonal blocks: wave w inverts block a = w of both value heads,
-             * column kc of U_aa on lane kc (+16 for head 1; lanes 32-63 repeat
-             * lanes 0-31 and do not write) */
-            {
-                const int a = w, v = (lane >> 4) & 1, kc = lane & 15;
-                const float *Md = MB + (v * 10 + blk_q(a, a)) * BLK;
-                float u[16];
-    #pragma unroll
-                for (int s = 15; s >= 0; s--) {
-                    float4 mrow[4];
-    #pragma unroll
-                    for (int q = 0; q < 4; q++) mrow[q] = *reinterpret_cast<const float4 *>(&Md[s * BS + 4 * q]);
-                    float acc = s == kc ? 1.0f : 0.0f;
-    #pragma unroll
-                    for (int r = s + 1; r < 16; r++) acc = fmaf(-el(mrow[r >> 2], r & 3), u[r], acc);
-                    u[s] = acc;
-                }
-                if (lane < 32) {
-                    float *Td = TB + (v * 10 + blk_q(a, a)) * BLK + kc * BS;     /* T_aa row kc */
-    #pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        *reinterpret_cast<float4 *>(&Td[4 * q]) = make_float4(u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]);
-                    float *Ud = UD + (v * 4 + a) * BLK;
-    #pragma unroll
-                    for (int s = 0; s < 16; s++) Ud[s * BS + kc] = u[s];
-                }
-            }
-            q35_lds_barrier();
+    /* diagonal blocks: wave w inverts block a = w of both value heads,
+     * column kc of U_aa on lane kc (+16 for head 1; lanes 32-63 repeat
+     * lanes 0-31 and do not write) */
+    if (NW == 4 || w < 4) {
+        const int a = w, v = (lane >> 4) & 1, kc = lane & 15;
+        const float *Md = MB + (v * 10 + blk_q(a, a)) * BLK;
+        float u[16];
+#pragma unroll
+        for (int s = 15; s >= 0; s--) {
+            float4 mrow[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) mrow[q] = *reinterpret_cast<const float4 *>(&Md[s * BS + 4 * q]);
+            float acc = s == kc ? 1.0f : 0.0f;
+#pragma unroll
+            for (int r = s + 1; r < 16; r++) acc = fmaf(-el(mrow[r >> 2], r & 3), u[r], acc);
+            u[s] = acc;
+        }
+        if (lane < 32) {
+            float *Td = TB + (v * 10 + blk_q(a, a)) * BLK + kc * BS;     /* T_aa row kc */
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<float4 *>(&Td[4 * q]) = make_float4(u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]);
+            float *Ud = UD + (v * 4 + a) * BLK;
+#pragma unroll
+            for (int s = 0; s < 16; s++) Ud[s * BS + kc] = u[s];
+        }
+    }
+    q35_lds_barrier();
 
-            /* off-diagonal blocks by distance d = b - a: jobs (head v, block a),
-             * dealt round-robin over the waves; each is two 16x16x16 products */
-    #pragma unroll
-            for (int d = 1; d < 4; d++) {
-                for (int j = w; j < 2 * (4 - d); j += 4) {
-                    const int v = j / (4 - d), a = j % (4 - d), b = a + d;
-                    f32x4_t wacc = {0.f, 0.f, 0.f, 0.f};
-                    for (int cb = a + 1; cb <= b; cb++) {
-                        /* X = M_ac row-major; Y = U_cb, read as its transpose T_bc */
-                        const float4 xa = *reinterpret_cast<const float4 *>(&MB[(v * 10 + blk_q(a, cb)) * BLK + l16 * BS + 4 * lq]);
-                        const float4 yb = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(cb, b)) * BLK + l16 * BS + 4 * lq]);
-    #pragma unroll
-                        for (int e = 0; e < 4; e++) wacc = mfma4(el(xa, e), el(yb, e), wacc);
-                    }
-                    /* T_ba = (-W^T) U_aa^T: this lane's W entries W[4lq+e][l16] are
-                     * X[l16][4lq+e] of -W^T as they stand; Y^T = U_aa row-major */
-                    const float4 ud = *reinterpret_cast<const float4 *>(&UD[(v * 4 + a) * BLK + l16 * BS + 4 * lq]);
-                    f32x4_t tb = {0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
-                    for (int e = 0; e < 4; e++) tb = mfma4(-wacc[e], el(ud, e), tb);
-                    float *Tt = TB + (v * 10 + blk_q(a, b)) * BLK;
-    #pragma unroll
-                    for (int i = 0; i < 4; i++) Tt[(4 * lq + i) * BS + l16] = tb[i];
-                }
-                q35_lds_barrier();
+    /* off-diagonal blocks by distance d = b - a: jobs (head v, block a),
+     * dealt round-robin over the waves; each is two 16x16x16 products */
+#pragma unroll
+    for (int d = 1; d < 4; d++) {
+        for (int j = w; j < 2 * (4 - d); j += NW) {
+            const int v = j / (4 - d), a = j % (4 - d), b = a + d;
+            f32x4_t wacc = {0.f, 0.f, 0.f, 0.f};
+            for (int cb = a + 1; cb <= b; cb++) {
+                /* X = M_ac row-major; Y = U_cb, read as its transpose T_bc */
+                const float4 xa = *reinterpret_cast<const float4 *>(&MB[(v * 10 + blk_q(a, cb)) * BLK + l16 * BS + 4 * lq]);
+                const float4 yb = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(cb, b)) * BLK + l16 * BS + 4 * lq]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) wacc = mfma4(el(xa, e), el(yb, e), wacc);
             }
+            /* T_ba = (-W^T) U_aa^T: this lane's W entries W[4lq+e][l16] are
+             * X[l16][4lq+e] of -W^T as they stand; Y^T = U_aa row-major */
+            const float4 ud = *reinterpret_cast<const float4 *>(&UD[(v * 4 + a) * BLK + l16 * BS + 4 * lq]);
+            f32x4_t tb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; e++) tb = mfma4(-wacc[e], el(ud, e), tb);
+            float *Tt = TB + (v * 10 + blk_q(a, b)) * BLK;
+#pragma unroll
+            for (int i = 0; i < 4; i++) Tt[(4 * lq + i) * BS + l16] = tb[i];
+        }
+        q35_lds_barrier();
+    }
 
-            /* T out: 2 heads x the 10 lower blocks x 16 rows x 4 float4, each wave
-             * instruction one whole 1 KB block */
-    #pragma unroll
-            for (int u = 0; u < 5; u++) {
-                const int idx = u * 256 + t, v = idx / 640, rem = idx % 640;
-                const int j = rem >> 6, r = (rem >> 2) & 15, q4 = rem & 3;
-                const int bb = j < 1 ? 0 : j < 3 ? 1 : j < 6 ? 2 : 3, ba = j - tri_idx(bb, 0);
-                const float4 o = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(ba, bb)) * BLK + r * BS + 4 * q4]);
-                *reinterpret_cast<float4 *>(p.T + ((size_t)c * VH + 2 * kh + v) * C * C + j * 256 + r * 16 + 4 * q4) = o;
-            }
+    /* T out: 2 heads x the 10 lower blocks x 16 rows x 4 float4, each wave
+     * instruction one whole 1 KB block */
+#pragma unroll
+    for (int u = 0; u < (1280 + 64 * NW - 1) / (64 * NW); u++) {
+        const int idx = u * 64 * NW + t, v = idx / 640, rem = idx % 640;
+        if (1280 % (64 * NW) != 0 && idx >= 1280) break;     /* wave-uniform */
+        const int j = rem >> 6, r = (rem >> 2) & 15, q4 = rem & 3;
+        const int bb = j < 1 ? 0 : j < 3 ? 1 : j < 6 ? 2 : 3, ba = j - tri_idx(bb, 0);
+        const float4 o = *reinterpret_cast<const float4 *>(&TB[(v * 10 + blk_q(ba, bb)) * BLK + r * BS + 4 * q4]);
+        *reinterpret_cast<float4 *>(p.T + ((size_t)c * VH + 2 * kh + v) * C * C + j * 256 + r * 16 + 4 * q4) = o;
+    }
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_kernel(Q35LinPrefill p) {
@@ -407,36 +409,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         q35_lds_barrier();
 
-        invert_blocks(p, MB, TB, UD, c, kh, w, t);
+        invert_blocks<4>(p, MB, TB, UD, c, kh, w, t);
         q35_lds_barrier();                       /* T read out: the next item may overwrite the LDS */
     }
 }
 
 /* ---- the two kernels before the scan in one launch, for few chunks -------- *
- * With few chunks conv_kernel and chunk_kernel are two short launches of
- * which each waits out its own memory round trips, and chunk_kernel's WG
- * count is 16 a chunk.  Here an item (chunk, key head) is three workgroups, each
- * convolving the raw rows of the heads it needs (64 + 3 rows, all loads ahead
- * of the first use; half-wave hw has tokens 8 hw .. + 7, 4 channels a lane):
- * role 0 K -> K K^T, T, the gate vectors; role 1 Q and K -> Q K^T, Pm; role 2
- * the two value heads.  K is convolved twice and the gates twice; nothing
- * passes through memory between the two steps.  The arithmetic is conv_kernel's
- * and chunk_kernel's, in their order: results are bit-identical. */
-__device__ __forceinline__ void conv_head(const Q35LinPrefill &p, int c, int grp, bool store, float *lds) {
-    const int t = threadIdx.x, hw = t >> 5, KH = p.k_heads, rows = 2 * KH * KD + p.v_heads * VD;
-    const int c0 = grp * KD + 4 * (t & 31), b0 = c * C, bb = b0 + 8 * hw;
-    const uint4 wa = *reinterpret_cast<const uint4 *>(p.conv_w + (size_t)c0 * 4);
-    const uint4 wb = *reinterpret_cast<const uint4 *>(p.conv_w + (size_t)c0 * 4 + 8);
+ * With few chunks conv_kernel and chunk_kernel are two short launches of a few
+ * workgroups, each waiting out its own memory round trips.  Here an item
+ * (chunk, key head) is three workgroups of 8 waves, each convolving the raw rows
+ * of the heads it needs (64 + 3 rows, all loads ahead of the first use; half-
+ * wave hw has tokens 4 hw .. + 3, 4 channels a lane): role 0 K -> K K^T, T;
+ * role 1 Q and K -> Q K^T, Pm, and the gate vectors; role 2 the two value
+ * heads.  K is convolved twice and the gates twice; nothing passes through
+ * memory between the two steps.  The arithmetic is conv_kernel's and
+ * chunk_kernel's, in their order: results are bit-identical.  What bounds it is
+ * role 0's chain: raw rows, conv, a tile's 32 dependent MFMAs, the triangular
+ * inverse. */
+constexpr int FEW_WAVES = 8, FEW_TOK = C / (2 * FEW_WAVES);
+struct ConvRows {
+    float4 x[FEW_TOK + 3];
+    uint4 wa, wb;
+};
+__device__ __forceinline__ void conv_load(ConvRows &R, const Q35LinPrefill &p, int c, int grp) {
+    const int t = threadIdx.x, hw = t >> 5, rows = 2 * p.k_heads * KD + p.v_heads * VD;
+    const int c0 = grp * KD + 4 * (t & 31), b0 = c * C, bb = b0 + FEW_TOK * hw;
     const int r0 = max(b0 - 3, 0);
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
         q35_uniform_ptr(const_cast<float *>(p.qkv) + (size_t)r0 * rows), 0, min(p.B - r0, C + 3) * rows * 4,
         Q35_BUF_DW3);
-    float4 xr[11];
+    R.wa = *reinterpret_cast<const uint4 *>(p.conv_w + (size_t)c0 * 4);
+    R.wb = *reinterpret_cast<const uint4 *>(p.conv_w + (size_t)c0 * 4 + 8);
 #pragma unroll
-    for (int k = 0; k < 11; k++) {
+    for (int k = 0; k < FEW_TOK + 3; k++) {
         const int b = bb - 3 + k;
-        xr[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                               rq, b >= 0 ? (uint32_t)(((b - r0) * rows + c0) * 4) : 0x80000000u, 0, 0));
+        R.x[k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rq, b >= 0 ? (uint32_t)(((b - r0) * rows + c0) * 4) : 0x80000000u, 0, 0));
     }
     if (c == 0) {                      /* the three rows before the batch: the ring */
         const __amdgpu_buffer_rsrc_t rr =
@@ -447,19 +455,25 @@ __device__ __forceinline__ void conv_head(const Q35LinPrefill &p, int c, int grp
             const float4 x = __builtin_bit_cast(
                 float4, __builtin_amdgcn_raw_buffer_load_b128(
                             rr, pp >= 0 ? (uint32_t)(((pp & 3) * rows + c0) * 4) : 0x80000000u, 0, 0));
-            if (hw == 0) xr[k] = x;
+            if (hw == 0) R.x[k] = x;
         }
     }
-    const uint2 wt[4] = {make_uint2(wa.x, wa.y), make_uint2(wa.z, wa.w), make_uint2(wb.x, wb.y),
-                         make_uint2(wb.z, wb.w)};
+}
+/* the head's rows to memory (store) and to the LDS tile lds (non-NULL; pad rows zero) */
+__device__ __forceinline__ void conv_rows(const ConvRows &R, const Q35LinPrefill &p, int c, int grp, bool store,
+                                          float *lds) {
+    const int t = threadIdx.x, hw = t >> 5, KH = p.k_heads, rows = 2 * KH * KD + p.v_heads * VD;
+    const int c0 = grp * KD + 4 * (t & 31), bb = c * C + FEW_TOK * hw;
+    const uint2 wt[4] = {make_uint2(R.wa.x, R.wa.y), make_uint2(R.wa.z, R.wa.w), make_uint2(R.wb.x, R.wb.y),
+                         make_uint2(R.wb.z, R.wb.w)};
     const float scale = grp < KH ? 1.0f / (float)KD : 1.0f / sqrtf((float)KD);
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
+    for (int j = 0; j < FEW_TOK; j++) {
         const int b = bb + j;
         float y[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const float x[4] = {el(xr[j], e), el(xr[j + 1], e), el(xr[j + 2], e), el(xr[j + 3], e)};
+            const float x[4] = {el(R.x[j], e), el(R.x[j + 1], e), el(R.x[j + 2], e), el(R.x[j + 3], e)};
             y[e] = q35_conv_silu_fast(x, wt[e], p.t0 + b);
         }
         if (grp < 2 * KH) {
@@ -473,45 +487,40 @@ __device__ __forceinline__ void conv_head(const Q35LinPrefill &p, int c, int grp
         const bool live = b < p.B;
         const float4 o = live ? make_float4(y[0], y[1], y[2], y[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
         if (store && live) *reinterpret_cast<float4 *>(p.post + (size_t)b * rows + c0) = o;
-        if (lds) *reinterpret_cast<float4 *>(&lds[sw128(8 * hw + j, 4 * (t & 31))]) = o;
+        if (lds) *reinterpret_cast<float4 *>(&lds[sw128(FEW_TOK * hw + j, 4 * (t & 31))]) = o;
     }
 }
 
-__global__ __launch_bounds__(256) void chunk_few_kernel(Q35LinPrefill p) {
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    __builtin_assume(w >= 0 && w < 4);
-    const int KH = p.k_heads, VH = p.v_heads, n_items = p.n_chunks * KH;
-    const int role = blockIdx.x / n_items, it = blockIdx.x % n_items;
-    const int c = it % p.n_chunks, kh = it / p.n_chunks;
-    const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, lq = lane >> 4;
-    __shared__ __align__(16) float sbuf[2 * C * KD];
-    __shared__ __align__(16) double sG[2][C];
-    __shared__ __align__(16) float sBeta[2][C];
-    float *sK = sbuf, *sQ = sbuf + C * KD;
-
-    if (role == 2) {
-        conv_head(p, c, 2 * KH + 2 * kh, true, nullptr);
-        conv_head(p, c, 2 * KH + 2 * kh + 1, true, nullptr);
-        return;
+/* the decayed lower tiles of K K^T (ROLE 0: A, as M blocks into LDS) or Q K^T
+ * (ROLE 1: Pm, to memory), chunk_kernel's tiles and order, on the first six
+ * waves; the last two do the gates meanwhile, from the inputs in gt */
+constexpr int TILE_WAVES = FEW_WAVES - 2;
+struct GateIn {
+    float a, b, A_log;
+    uint16_t dt;
+};
+__device__ __forceinline__ GateIn gates_load(const Q35LinPrefill &p, int c, int kh, int w) {
+    const int h = 2 * kh + (w & 1), b = min(c * C + (int)(threadIdx.x & 63), p.B - 1);
+    return GateIn{p.a[(size_t)b * p.v_heads + h], p.b[(size_t)b * p.v_heads + h], p.A_log[h], p.dt_bias[h]};
+}
+template <int ROLE>
+__device__ __forceinline__ void few_tiles(const Q35LinPrefill &p, int c, int kh, int w, const GateIn &gt,
+                                          float *sbuf, double (*sG)[C], float (*sBeta)[C]) {
+    const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, lq = lane >> 4, VH = p.v_heads;
+    const float *sK = sbuf, *X = ROLE == 0 ? sbuf : sbuf + C * KD;
+    if (w >= TILE_WAVES) {
+        const int v = w & 1;
+        float g, beta;
+        q35_lin_gates(gt.a, gt.b, gt.A_log, gt.dt, &g, &beta);
+        if (c * C + lane >= p.B) g = beta = 0.f;
+        decay_vectors(p, sG[v], sBeta[v], c, 2 * kh + v, lane, g, beta, ROLE == 1);
     }
-    conv_head(p, c, KH + kh, role == 0, sK);
-    if (role == 1) conv_head(p, c, kh, true, sQ);
-    if (w < 2) {
-        const int h = 2 * kh + w, b = c * C + lane;
-        float g = 0.f, beta = 0.f;
-        if (b < p.B)
-            q35_lin_gates(p.a[(size_t)b * VH + h], p.b[(size_t)b * VH + h], p.A_log[h], p.dt_bias[h], &g, &beta);
-        decay_vectors(p, sG[w], sBeta[w], c, h, lane, g, beta, role == 0);
-    }
-    q35_lds_barrier();
-
-    /* the 10 lower 16x16 tiles of K K^T (role 0) or Q K^T, as chunk_kernel's */
-    const float *X = role == 0 ? sK : sQ;
-    f32x4_t res[3];
+    constexpr int NT = 2;                        /* tiles w and w + 6 of 10 */
+    f32x4_t res[NT];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const int m = w + 4 * k;
-        if (m >= 10) break;
+    for (int k = 0; k < NT; k++) {
+        const int m = w + TILE_WAVES * k;
+        if (w >= TILE_WAVES || m >= 10) break;   /* wave-uniform */
         const int tr = m < 1 ? 0 : m < 3 ? 1 : m < 6 ? 2 : 3;
         const int tc = m - (tr * (tr + 1)) / 2;
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -524,28 +533,37 @@ __global__ __launch_bounds__(256) void chunk_few_kernel(Q35LinPrefill p) {
         }
         res[k] = acc;
     }
-    q35_lds_barrier();                           /* K no longer read */
-    float *MB = sbuf, *TB = sbuf + 2 * 10 * BLK, *UD = sbuf + 4 * 10 * BLK;
+    q35_lds_barrier();                           /* K no longer read; the gates in LDS */
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const int m = w + 4 * k;
-        if (m >= 10) break;
+    for (int k = 0; k < NT; k++) {
+        const int m = w + TILE_WAVES * k;
+        if (w >= TILE_WAVES || m >= 10) break;
         const int tr = m < 1 ? 0 : m < 3 ? 1 : m < 6 ? 2 : 3;
         const int tc = m - (tr * (tr + 1)) / 2;
         const int s = 16 * tc + l16, r0 = 16 * tr + 4 * lq;
 #pragma unroll
         for (int v = 0; v < 2; v++) {
             const double gs = sG[v][s];
+            const double2 g01 = *reinterpret_cast<const double2 *>(&sG[v][r0]);
+            const double2 g23 = *reinterpret_cast<const double2 *>(&sG[v][r0 + 2]);
+            const float4 bt = *reinterpret_cast<const float4 *>(&sBeta[v][r0]);
+            const double gr[4] = {g01.x, g01.y, g23.x, g23.y};
+            const float br[4] = {bt.x, bt.y, bt.z, bt.w};
             float o[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int r = r0 + i;
-                const float dec = __expf((float)(sG[v][r] - gs));
-                const float av = sBeta[v][r] * dec * res[k][i], pv = dec * res[k][i];
-                o[i] = role == 0 ? (s < r ? av : 0.0f) : (s <= r ? pv : 0.0f);
+                const float dec = __expf((float)(gr[i] - gs));   /* v_exp_f32, ~1 ulp */
+                if constexpr (ROLE == 0) {
+                    const float av = br[i] * dec * res[k][i];
+                    o[i] = s < r ? av : 0.0f;
+                } else {
+                    const float pv = dec * res[k][i];
+                    o[i] = s <= r ? pv : 0.0f;
+                }
             }
-            if (role == 0) {
-                *reinterpret_cast<float4 *>(&MB[(v * 10 + blk_q(tc, tr)) * BLK + l16 * BS + 4 * lq]) =
+            if constexpr (ROLE == 0) {
+                *reinterpret_cast<float4 *>(&sbuf[(v * 10 + blk_q(tc, tr)) * BLK + l16 * BS + 4 * lq]) =
                     make_float4(o[0], o[1], o[2], o[3]);
             } else {
                 float *Pm = p.Pm + ((size_t)c * VH + 2 * kh + v) * C * C + tri_idx(tr, tc) * 256;
@@ -554,9 +572,42 @@ __global__ __launch_bounds__(256) void chunk_few_kernel(Q35LinPrefill p) {
             }
         }
     }
-    if (role == 1) return;
-    q35_lds_barrier();
-    invert_blocks(p, MB, TB, UD, c, kh, w, t);
+}
+
+__global__ __launch_bounds__(64 * FEW_WAVES) void chunk_few_kernel(Q35LinPrefill p) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __builtin_assume(w >= 0 && w < FEW_WAVES);
+    const int KH = p.k_heads, n_items = p.n_chunks * KH;
+    const int role = blockIdx.x / n_items, it = blockIdx.x % n_items;
+    const int c = it % p.n_chunks, kh = it / p.n_chunks;
+    __shared__ __align__(16) float sbuf[2 * C * KD];
+    __shared__ __align__(16) double sG[2][C];
+    __shared__ __align__(16) float sBeta[2][C];
+
+    ConvRows R0, R1;
+    GateIn gt = {};
+    if (role < 2 && w >= TILE_WAVES) gt = gates_load(p, c, kh, w);
+    if (role == 0) {
+        conv_load(R0, p, c, KH + kh);
+        conv_rows(R0, p, c, KH + kh, true, sbuf);
+        q35_lds_barrier();
+        few_tiles<0>(p, c, kh, w, gt, sbuf, sG, sBeta);
+        q35_lds_barrier();
+        invert_blocks<FEW_WAVES>(p, sbuf, sbuf + 2 * 10 * BLK, sbuf + 4 * 10 * BLK, c, kh, w, threadIdx.x);
+    } else if (role == 1) {
+        conv_load(R0, p, c, KH + kh);
+        conv_load(R1, p, c, kh);
+        conv_rows(R0, p, c, KH + kh, false, sbuf);
+        conv_rows(R1, p, c, kh, true, sbuf + C * KD);
+        q35_lds_barrier();
+        few_tiles<1>(p, c, kh, w, gt, sbuf, sG, sBeta);
+    } else {
+        const int v0 = 2 * KH + 2 * kh;
+        conv_load(R0, p, c, v0);
+        conv_load(R1, p, c, v0 + 1);
+        conv_rows(R0, p, c, v0, true, nullptr);
+        conv_rows(R1, p, c, v0 + 1, true, nullptr);
+    }
 }
 
 /* ---- 4. sequential scan over chunks per (value head, 16-column block) ---- *
@@ -1028,7 +1079,7 @@ extern "C" hipError_t q35_lin_prefill(const Q35LinPrefill *pin, hipStream_t stre
     if (p.xw && (p.mpad < p.B || p.mpad % Q35_XW_ROWS != 0 || !p.xsum)) return hipErrorInvalidValue;
     hipError_t e;
     if (p.B <= FEW_TOKENS) {
-        hipLaunchKernelGGL(chunk_few_kernel, dim3(3 * p.n_chunks * p.k_heads), dim3(256), 0, stream, p);
+        hipLaunchKernelGGL(chunk_few_kernel, dim3(3 * p.n_chunks * p.k_heads), dim3(64 * FEW_WAVES), 0, stream, p);
     } else {
         hipLaunchKernelGGL(conv_kernel, dim3(rows / 1024, (p.B + CT - 1) / CT), dim3(256), 0, stream, p);
         if ((e = hipGetLastError()) != hipSuccess) return e;
