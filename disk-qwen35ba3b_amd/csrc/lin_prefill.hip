@@ -989,7 +989,11 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_kernel(Q35LinPrefill p) {
  * A lane of that operand is 32 columns of a row, so the wave's rows pass
  * through its own LDS area and lane (token l % TT, quarter l / TT of the
  * head) stores the digits, 16 TT consecutive bytes a quarter. */
-constexpr int FEW_TOKENS = 1024;
+/* us a call, conv_kernel + chunk_kernel | chunk_few_kernel: 64 tokens 25.9 |
+ * 18.4, 256 39.9 | 32.8, 1024 80.8 | 72.4, 1500 113.7 | 103.7, 3000 207 |
+ * 204, 4096 276 | 283 (the second conv of K and the idle waves of the
+ * inverse cost more than the launch) */
+constexpr int FEW_TOKENS = 3072;
 constexpr int GTT = 4;
 template <int TT, bool XW>
 __global__ __launch_bounds__(256) void gnorm_kernel(Q35LinPrefill p) {
