@@ -22,7 +22,7 @@
  * The new token (position `token`) is attended in fp32 from registers (as
  * the reference does with its fp32 cache) by the last chunk's workgroup,
  * which also writes the bf16 cache row.
- * Kernel 2 (merge): rescales and sums the P partials of each q head and
+ * Kernel 2 (merge; not launched for a single chunk): rescales and sums the P partials of each q head and
  * applies the gate, one wave per (head, 16 dims) with wave reductions only.
  *
  * Every global input of the prologue is loaded up front so the workgroup
@@ -162,18 +162,22 @@ __device__ __forceinline__ void attend_tile(KTile &kt, VTile &vt, const bf16x8_t
 /* The arguments are scalars, not the struct, so that the first nine (14
  * dwords: what the prologue and the first K/V tiles need) are preloaded
  * into SGPRs at wave launch (-amdgpu-kernarg-preload-count=9 for this
- * file); the rest load while those loads are in flight. */
+ * file); the rest load while those loads are in flight.
+ * ONE: a single chunk; the workgroup's merged heads are the result, and go
+ * out gated (attn_out) with no partials and no merge launch. */
+template <bool ONE>
 __global__ __launch_bounds__(NT) void gqa_split_kernel(int token, int t_tiles, int chunk, int n_chunks,
                                                        const float *q_gate, const uint16_t *qn_w,
                                                        const float *rope, uint16_t *kt, uint16_t *vt,
                                                        const float *k_new, const float *v_new,
                                                        const uint16_t *kn_w, float *part_o, float *part_ml,
-                                                       float *k_post, int heads, int kv_heads) {
+                                                       float *k_post, int heads, int kv_heads,
+                                                       float *attn_out) {
     Q35GqaDecode p;
     p.token = token, p.t_tiles = t_tiles, p.chunk = chunk, p.n_chunks = n_chunks;
     p.q_gate = q_gate, p.qn_w = qn_w, p.rope = rope, p.kt = kt, p.vt = vt;
     p.k_new = k_new, p.v_new = v_new, p.kn_w = kn_w, p.part_o = part_o, p.part_ml = part_ml;
-    p.k_post = k_post, p.heads = heads, p.kv_heads = kv_heads, p.attn_out = nullptr;
+    p.k_post = k_post, p.heads = heads, p.kv_heads = kv_heads, p.attn_out = attn_out;
     const int c = blockIdx.x, g = blockIdx.y;
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
     const int n_past = p.token;
@@ -226,6 +230,8 @@ __global__ __launch_bounds__(NT) void gqa_split_kernel(int token, int t_tiles, i
     VTile va;
     load_k(ka, krs, wv * 8192 + koff);
     load_v(va, vrs, wv * 8192 + voff);
+    float4 gate = make_float4(0.f, 0.f, 0.f, 0.f);      /* of head w, which wave w merges */
+    if constexpr (ONE) gate = *reinterpret_cast<const float4 *>(p.q_gate + ((size_t)(g * G + w) * 2 + 1) * D + d0);
 
     /* q of heads HPW*w .. HPW*w+HPW-1 (of this kv head): norm + RoPE, then straight into
      * the MFMA B-operand layout: entry [kk][lane'] holds 8 bf16 of column
@@ -361,6 +367,18 @@ __global__ __launch_bounds__(NT) void gqa_split_kernel(int token, int t_tiles, i
             o.z = fmaf(v.z, f, o.z);
             o.w = fmaf(v.w, f, o.w);
         }
+        if constexpr (ONE) {
+            const float ri = __builtin_amdgcn_rcpf(L);
+            o.x = o.x * ri * q35_sigmoid_fast(gate.x);
+            o.y = o.y * ri * q35_sigmoid_fast(gate.y);
+            o.z = o.z * ri * q35_sigmoid_fast(gate.z);
+            o.w = o.w * ri * q35_sigmoid_fast(gate.w);
+            __builtin_amdgcn_raw_buffer_store_b128(
+                __builtin_bit_cast(u32x4_t, o),
+                __builtin_amdgcn_make_buffer_rsrc(q35_uniform_ptr(p.attn_out), 0, p.heads * D * 4, Q35_BUF_DW3),
+                ((g * G + hh) * D + d4) * 4, 0, Q35_ST_SC1);
+            return;
+        }
         const __amdgpu_buffer_rsrc_t ors =
             __builtin_amdgcn_make_buffer_rsrc(q35_uniform_ptr(po), 0, G * D * 4, Q35_BUF_DW3);
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o), ors, (hh * D + d4) * 4, 0,
@@ -474,14 +492,21 @@ __global__ __launch_bounds__(64) void gqa_merge_kernel(int n_chunks, int heads, 
 }  // namespace
 
 extern "C" void q35_gqa_split(int n_past, int *chunk, int *n_chunks) {
+    /* up to 256 positions: one chunk a kv head, with no merge launch (us a
+     * call, 64-position chunks and a merge -> one chunk: 1 position 8.2 -> 6.4, 128 8.2 ->
+     * 6.5, 200 8.2 -> 8.0, 256 8.2 -> 7.5; a third tile a wave would cost what
+     * the merge does) */
+    if (n_past <= 256) {
+        *chunk = 256;
+        *n_chunks = 1;
+        return;
+    }
     /* about 128 chunks per kv head (256 workgroups); chunks are multiples of
      * 64 positions (4 sub-tiles per wave at least) */
     const int target = 128;
     int per = (n_past + target - 1) / target;
     int ch = ((per + 63) / 64) * 64;
-    if (ch < 64) ch = 64;
-    int P = (n_past + ch - 1) / ch;
-    if (P < 1) P = 1;
+    const int P = (n_past + ch - 1) / ch;
     *chunk = ch;
     *n_chunks = P;
 }
@@ -491,11 +516,12 @@ extern "C" int q35_gqa_max_chunks(void) { return MAX_CHUNKS; }
 extern "C" hipError_t q35_gqa_decode(const Q35GqaDecode *p, hipStream_t stream) {
     if (p->heads != p->kv_heads * G || p->n_chunks < 1 || p->n_chunks > MAX_CHUNKS)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(gqa_split_kernel, dim3(p->n_chunks, p->kv_heads), dim3(NT), 0, stream, p->token,
+    const auto split = p->n_chunks == 1 ? gqa_split_kernel<true> : gqa_split_kernel<false>;
+    hipLaunchKernelGGL(split, dim3(p->n_chunks, p->kv_heads), dim3(NT), 0, stream, p->token,
                        p->t_tiles, p->chunk, p->n_chunks, p->q_gate, p->qn_w, p->rope, p->kt, p->vt, p->k_new,
-                       p->v_new, p->kn_w, p->part_o, p->part_ml, p->k_post, p->heads, p->kv_heads);
+                       p->v_new, p->kn_w, p->part_o, p->part_ml, p->k_post, p->heads, p->kv_heads, p->attn_out);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || p->n_chunks == 1) return e;
     if (p->n_chunks <= 128)
         hipLaunchKernelGGL(gqa_merge_kernel<2>, dim3(p->heads, D / 16), dim3(64), 0, stream, p->n_chunks,
                            p->heads, p->part_ml, p->part_o, p->q_gate, p->attn_out);

@@ -197,6 +197,13 @@ def test_gqa_decode_step(n_past):
     ga.close()
 
 
+@pytest.mark.parametrize("n_past", [127, 128, 129, 241, 255, 256, 257])
+def test_gqa_decode_one_chunk_edges(n_past):
+    """One tile a wave and two, a ragged last tile, and both sides of the line up to
+    which one workgroup a kv head stores the gated result itself."""
+    test_gqa_decode_step(n_past)
+
+
 def test_gqa_decode_consecutive_steps():
     """64 steps from 500 past rows.  The device cache holds bf16 rows, so the
     oracle's cache gets each new row bf16-rounded too (same inputs); the
