@@ -187,15 +187,17 @@ __global__ void wt_kernel(const uint32_t *vals, u32x4_t *wt, int N, int K, int64
         const u32x4_t v =
             *reinterpret_cast<const u32x4_t *>(vals + (size_t)row * (K / 8) + 8 * g + 4 * wslot(r, p & 1));
 #pragma unroll
-        for (int f = 0; f < 32; f++) {
-            const int k = q35_xw_col(f);
-            const uint32_t q = (v[k >> 3] >> (4 * (k & 7))) & 15u;
+        for (int u = 0; u < 2; u++) {               /* fields 16 u .. + 15: 96 bits */
+            uint32_t d[3] = {0u, 0u, 0u};
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int pos = 6 * (f & 15) + j, b = pos & 31;
-                const int src = pos < 32 ? 0 : pos < 64 ? 1 : (int)((M0 >> b) & 1);
-                o[2 * (f >> 4) + src] |= ((q >> j) & 1u) << b;
+            for (int f = 0; f < 16; f++) {
+                const int k = q35_xw_col(16 * u + f), pos = 6 * f, b = pos & 31;
+                const uint32_t q = (v[k >> 3] >> (4 * (k & 7))) & 15u;
+                d[pos >> 5] |= q << b;
+                if (b > 28) d[(pos >> 5) + 1] |= q >> (32 - b);
             }
+            o[2 * u] = (d[0] & M0) | (d[2] & ~M0);
+            o[2 * u + 1] = (d[1] & M1) | (d[2] & ~M1);
         }
     }
     wt[i] = o;
