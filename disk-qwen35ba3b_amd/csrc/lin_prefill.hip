@@ -27,13 +27,14 @@
  *                on fp32 MFMA (shared by the key head's two value heads),
  *                then per value head A, Pm, the decay vectors and T by
  *                16x16 blocks (diagonal blocks by back substitution, the
- *                rest on fp32 MFMA); the last chunk's workgroups also write
- *                the last min(B, 4) raw rows into the conv ring
+ *                rest on fp32 MFMA)
+ *                (few tokens: both as one launch, chunk_few_kernel)
  *   scan_kernel  per (value head, 16-column block of vd), sequential over
  *                chunks: the state block stays in LDS; K S0, Q S0, Delta,
  *                O and S_end on fp32 MFMA (v_mfma_f32_16x16x4_f32); O
- *                unnormalised into out
- *   gnorm_kernel per (4 tokens, value head): RMSNormGated of out with z
+ *                unnormalised into out; writes the last min(B, 4) raw rows
+ *                into the conv ring
+ *   gnorm_kernel per (4 or 16 tokens, value head): RMSNormGated of out with z
  *                (src/attn_qwen.c:726-749)
  * All arithmetic is fp32 (MFMA fp32 products are exact, accumulation fp32);
  * the conv's SiLU and norm reciprocal, the chunk's decay factors and the
