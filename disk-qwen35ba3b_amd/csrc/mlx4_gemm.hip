@@ -785,11 +785,12 @@ extern "C" hipError_t q35_mlx4_xprep(const Q35Mlx4Xprep *p, hipStream_t stream) 
         (int64_t)8 * p->ldx * 4 >= ((int64_t)1 << 31))
         return hipErrorInvalidValue;
     /* us a launch at XR = 2 | 4 | 8 (K = 2048; K = 4096):
-     *   M =   64:  2.9 |  3.8 |  5.5;   3.0 |  4.6 |  8.1
-     *   M =  256:  3.5 |  4.0 |  5.7;   4.4 |  5.1 |  8.5
-     *   M = 1024:  6.3 |  4.9 |  6.5;  10.0 |  7.9 | 10.3
-     *   M = 2048: 10.3 |  7.5 |  8.2;  19.1 | 12.7 | 11.6
-     *   M = 4096: 19.4 | 12.6 | 11.6;  36.7 | 23.0 | 21.5 */
+     *   M =   64:  3.9 |  4.3 |  5.7;   4.8 |  5.8 |  8.6
+     *   M =  256:  4.5 |  4.5 |  5.9;   6.0 |  6.4 |  9.0
+     *   M =  512:  5.4 |  4.9 |  6.1;   8.2 |  7.2 |  9.9
+     *   M = 1024:  7.9 |  5.7 |  7.0;  12.8 |  9.4 | 11.2
+     *   M = 2048: 12.8 |  8.2 |  8.0;  24.2 | 13.4 | 12.9
+     *   M = 4096: 24.3 | 13.5 | 11.7;  47.1 | 26.3 | 25.4 */
     if (p->M <= 256)
         launch_xprep<2>(p, stream);
     else if (p->M <= 2048)
@@ -804,7 +805,7 @@ extern "C" hipError_t q35_mlx4_gemm(const Q35Mlx4Gemm *p, hipStream_t stream) {
         p->njobs > Q35_GEMM_MAX_JOBS || (int64_t)p->Mpad * p->K * 4 >= ((int64_t)1 << 31) ||
         (int64_t)(p->K / 64) * p->Mpad * 4 >= ((int64_t)1 << 31))
         return hipErrorInvalidValue;
-    /* buffer offsets are 32-bit: each weight and its (s, b') table below 2 GB */
+    /* buffer offsets are 32-bit: each weight and its scale / bias table below 2 GB */
     int64_t tiles = 0;
     for (int j = 0; j < p->njobs; j++) {
         const Q35Mlx4GemmJob *J = &p->jobs[j];
